@@ -850,8 +850,8 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
     }
 }
 
-// Plain per-output kernel for fp32 activations and unaligned shapes: one
-// thread per output; the dequantized weight is rounded to the activation dtype
+// Plain per-output kernel for shapes and alignments the MFMA kernels do not
+// take (launch_gemm_simple): one thread per output; the dequantized weight is rounded to the activation dtype
 // when round_dequant != 0 (GEMM semantics) and exact otherwise (GEMV).
 template <typename T, int EPI>
 __global__ void gemm_simple_kernel(GemmArgs a) {
@@ -1136,6 +1136,7 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs& a) {
 
 hipError_t launch_gemm_simple(hipStream_t s, const GemmArgs& a) {
     if (a.M == 0 || a.N == 0) return hipSuccess;
+    if (gemm_f32_takes(a)) return launch_gemm_f32(s, a);
     dim3 grid((a.N + 255) / 256, a.M);
     auto go = [&](auto tag) {
         using T = decltype(tag);

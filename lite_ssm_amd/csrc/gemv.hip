@@ -1097,6 +1097,12 @@ hipError_t gemv_plain(hipStream_t s, const GemvArgs& a) {
         hipError_t err = hipSuccess;
         if (launch_gemv_mma(s, a, err)) return err;
     }
+    if constexpr (__is_same(T, float)) {
+        // fp32 rows past the GEMV's own four: one fp32 GEMM over the weights
+        // instead of a launch per four rows (the two rules agree in fp32)
+        GemmArgs g{a.x, a.x_stride, a.w, a.s, a.y, a.y_stride, a.res, a.M, a.N, a.K, a.wfmt, a.act, a.epi, 0};
+        if (!a.norm_w && a.M > 4 && gemm_f32_takes(g)) return launch_gemm_f32(s, g);
+    }
     const int mrmax = rows_for<T>(c0, a.wfmt, a.norm_w ? 1 : 0);
     if (mrmax < 1) return hipErrorInvalidValue;
     for (uint32_t m0 = 0; m0 < a.M; m0 += (uint32_t)mrmax) {

@@ -217,8 +217,13 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs& a);
 // through lssm_linear (no workspace) measures 23.9 us unsplit against 26.5 us
 // split, so the generic entry keeps the single launch.
 constexpr size_t GEMM_WS_FLOATS = (size_t)8 << 20;   // 32 MiB
-// Simple fp32 (or any dtype) reference-layout GEMM used for F32 activations.
+// GEMM for fp32 activations (any row count) and for operands the MFMA GEMMs'
+// 16-byte loads cannot take: fp32 on the fp32 MFMA where gemm_f32_takes says
+// so, else one thread per output.
 hipError_t launch_gemm_simple(hipStream_t s, const GemmArgs& a);
+// fp32 MFMA GEMM (gemm_f32.hip): K a multiple of 32, 16-byte aligned rows.
+bool gemm_f32_takes(const GemmArgs& a);
+hipError_t launch_gemm_f32(hipStream_t s, const GemmArgs& a);
 
 // SSD.  Strides are row strides in elements of the [.., L, ...] tensors.
 struct SsdArgs {

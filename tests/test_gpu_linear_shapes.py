@@ -1,0 +1,63 @@
+"""Linear kernels at the edges of their tiles: each dispatch branch at the row
+counts, widths and depths where it can go wrong, against the CPU oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+from gpu_util import act_host, assert_close, dev, empty
+
+pytestmark = pytest.mark.gpu
+
+ALL_FMTS = [O.W_DENSE, O.W_Q4_B32, O.W_Q4_G64, O.W_Q8_G32]
+
+
+def _weights(rng, N, K, wfmt, act, std=0.02):
+    wf = (rng.standard_normal((N, K)) * std).astype(np.float16).astype(np.float32)
+    return (O.to_act(wf, act), None) if wfmt == O.W_DENSE else O.quantize(wf, wfmt)
+
+
+def _sdev(s):
+    return None if s is None else dev(s)
+
+
+# --------------------------------------------------------------------------- fp32 GEMM
+# Up to 256 tiles of 32 x 32: eight waves split K (steps of 256, which end in
+# zeros for the K here); 70 x 6000 and 63 x 15970: 64 x 64 tiles; 300 x 3352
+# and 33 x 8150: 32 x 64.  Partial tiles in M and N.
+@pytest.mark.parametrize("wfmt", ALL_FMTS)
+@pytest.mark.parametrize("M,N,K", [(5, 1, 64), (33, 31, 192), (64, 200, 832), (65, 64, 64), (70, 6000, 192),
+                                   (33, 8150, 192), (63, 15970, 64), (300, 3352, 768)])
+def test_fp32_gemm_vs_oracle(ctx, rng, wfmt, M, N, K):
+    print(f"case: fp32 GEMM {wfmt} {M} x {N} x {K}", flush=True)
+    x = O.to_act(rng.standard_normal((M, K)), O.F32)
+    w, s = _weights(rng, N, K, wfmt, O.F32)
+    y = empty((M, N), O.F32)
+    ctx.linear(dev(x), dev(w), _sdev(s), y, M, N, K, wfmt, O.F32)
+    ref = O.linear(x, w, s, M, N, K, wfmt, O.F32, round_dequant=1)
+    # fp32 products and sums: K roundings of partial sums of a few outputs' size
+    assert_close(act_host(y, O.F32), ref, O.F32, 1e-5, "fp32 gemm")
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 96, 32), (40, 96, 96)])
+def test_fp32_gemm_dense_short_k_strides_epilogues(ctx, rng, M, N, K):
+    """K of 32 and 96 (dense and group-32 only), padded rows in and out, SiLU
+    and the in-place residual."""
+    import lite_ssm_amd as L
+    for wfmt in (O.W_DENSE, O.W_Q8_G32):
+        print(f"case: fp32 GEMM strided {wfmt} {M} x {N} x {K}", flush=True)
+        xp = rng.standard_normal((M, K + 4)).astype(np.float32)
+        x = np.ascontiguousarray(xp[:, :K])
+        w, s = _weights(rng, N, K, wfmt, O.F32)
+        res = rng.standard_normal((M, N + 3)).astype(np.float32)
+        y = dev(res)
+        ctx.linear(dev(xp), dev(w), _sdev(s), y, M, N, K, wfmt, O.F32, epi=L.EPI_ADD, residual=y,
+                   x_stride=K + 4, y_stride=N + 3)
+        ref = O.linear(O.to_act(x, O.F32), w, s, M, N, K, wfmt, O.F32, epi=O.EPI_ADD,
+                       residual=np.ascontiguousarray(res[:, :N]), round_dequant=1)
+        got = act_host(y, O.F32)
+        assert_close(np.ascontiguousarray(got[:, :N]), ref, O.F32, 1e-5, "add")
+        assert np.array_equal(got[:, N:], res[:, N:])          # the padding is left alone
+        y2 = empty((M, N), O.F32)
+        ctx.linear(dev(x), dev(w), _sdev(s), y2, M, N, K, wfmt, O.F32, epi=L.EPI_SILU)
+        ref = O.linear(O.to_act(x, O.F32), w, s, M, N, K, wfmt, O.F32, epi=O.EPI_SILU, round_dequant=1)
+        assert_close(act_host(y2, O.F32), ref, O.F32, 1e-5, "silu")
