@@ -34,6 +34,20 @@ bool gemm_ok(const void* x, uint32_t x_stride, const void* w, uint32_t K, int ac
     return act != LSSM_F32 && K % 64 == 0 && x_stride % 8 == 0 && al16(x) && al16(w);
 }
 
+// Decode batches whose x is packed once into the context's buffer for the
+// batched GEMV.
+bool pack_rows_ok(const lssm_ctx* ctx, const GemvArgs& g) {
+    return g.norm_w && ctx->xpack && gemv_rows_pays(g.M, g.N, g.K, g.wfmt, g.act) && al16(g.x) &&
+           al16(g.norm_w) && al16(g.w) && (g.wfmt == LSSM_W_DENSE || (uintptr_t)g.s % 4 == 0) && g.x_stride % 8 == 0;
+}
+hipError_t pack_rows(lssm_ctx* ctx, GemvArgs& g) {
+    const hipError_t e = launch_mma_pack(ctx->stream, g.x, g.x_stride, g.norm_w, g.eps, g.M, g.K, g.wfmt, g.act,
+                                         ctx->xpack);
+    g.xpack = ctx->xpack;
+    g.xrows = true;
+    return e;
+}
+
 int check_fmt_k(uint32_t K, int wfmt, const void* s) {
     LSSM_REQUIRE(valid_wfmt(wfmt), "linear: unknown weight format %d", wfmt);
     if (wfmt != LSSM_W_DENSE) {
@@ -123,7 +137,16 @@ int lssm_norm_linear_decode(lssm_ctx* ctx, const void* x, const void* norm_w, fl
     LSSM_REQUIRE(x && norm_w && w && y, "norm_linear_decode: null pointer");
     LSSM_REQUIRE(gemv_ok(w, K, wfmt, act), "norm_linear_decode: unsupported K / weight alignment");
     GemvArgs g{x, K, w, w_scales, y, N, residual, norm_w, eps, rows, N, K, wfmt, act, epi};
-    hipError_t e = launch_gemv(ctx->stream, g);
+    hipError_t e;
+    if (rows > 4 && dense_head_gemm(N, K, wfmt, act) && al16(x) && al16(norm_w)) {
+        // an lm_head: norm launch, then the tiled GEMM (dense: one rule)
+        e = launch_rmsnorm(ctx->stream, x, K, norm_w, ctx->xpack, K, rows, K, eps, act);
+        GemmArgs m{ctx->xpack, K, w, nullptr, y, N, residual, rows, N, K, wfmt, act, epi, 1};
+        if (e == hipSuccess) e = launch_gemm(ctx->stream, m);
+    } else {
+        e = pack_rows_ok(ctx, g) ? pack_rows(ctx, g) : hipSuccess;
+        if (e == hipSuccess) e = launch_gemv(ctx->stream, g);
+    }
     if (e != hipSuccess) return set_error(LSSM_EDEVICE, "norm_linear_decode: %s", hipGetErrorString(e));
     return finish(ctx, "norm_linear_decode");
 }
@@ -314,7 +337,8 @@ int lssm_inproj_decode(lssm_ctx* ctx, const void* hidden, const void* norm_w, co
     a.z = z;
     a.xbc_act = xbc_act;
     a.dt = dt;
-    hipError_t e = launch_inproj_decode(ctx->stream, a);
+    hipError_t e = pack_rows_ok(ctx, a.g) ? pack_rows(ctx, a.g) : hipSuccess;
+    if (e == hipSuccess) e = launch_inproj_decode(ctx->stream, a);
     if (e != hipSuccess) return set_error(LSSM_EDEVICE, "inproj_decode: %s", hipGetErrorString(e));
     return finish(ctx, "inproj_decode");
 }

@@ -136,7 +136,11 @@ struct lssm_engine {
     uint64_t* xfer_b = nullptr;
     uint32_t xfer_b_rows = 0;
     bool fuse_ssd_b = false;
-    // decode batches from this many rows pack x once per linear (launch_mma_pack);
+    // every weight and norm pointer is aligned as gemv_rows and its pack
+    // launch need it (16 bytes, scales 4)
+    bool rows_aligned = false;
+    // decode batches from this many rows pack x once per linear for the
+    // single-pass MFMA GEMV (launch_mma_pack);
     // LSSM_PACK_MIN_ROWS at creation overrides it; parts_min_rows is the same
     // for the normalise-on-load path below (LSSM_PARTS_MIN_ROWS)
     uint32_t pack_min_rows = 8;
@@ -254,6 +258,14 @@ struct lssm_engine {
                 if (e != hipErrorNotSupported) return e;
             }
             e = launch_gemv(st(), g);
+        } else if (rows_aligned && gemv_rows_pays(rows, vocab, d_model, LSSM_W_DENSE, act)) {
+            // norm_f into the packed rows, W streamed once
+            e = launch_mma_pack(st(), x, xs, norm_f, RMS_EPS, rows, d_model, LSSM_W_DENSE, act, d_gn);
+            GemvArgs g{x, xs, lm_head, nullptr, logits, vocab, nullptr, norm_f, RMS_EPS, rows, vocab,
+                       d_model, LSSM_W_DENSE, act, LSSM_EPI_NONE};
+            g.xpack = d_gn;
+            g.xrows = true;
+            if (e == hipSuccess) e = launch_gemv(st(), g);
         } else {
             e = launch_rmsnorm(st(), x, xs, norm_f, d_normed, d_model, rows, d_model, RMS_EPS, act);
             if (e == hipSuccess)
@@ -266,30 +278,31 @@ struct lssm_engine {
 
     // One decode step: ids -> next (all on device).  mamba2_block.cpp:317-327.
     hipError_t decode(const int32_t* ids, uint32_t B, int32_t* next) const {
-        // fused RMSNorm + linear kernels: the VALU GEMV up to 4 rows, the MFMA
-        // GEMV for decode batches of the shapes it takes
-        const bool fused_in = (B <= 4 && (int)B <= gemv_max_rows(d_model, wfmt, act)) ||
-                              (B >= 2 && gemv_mma_takes(B, proj, d_model, wfmt, act));
-        const bool fused_out = (B <= 4 && gemv_max_rows(d_inner, wfmt, act) >= 1) ||
-                               (B >= 2 && gemv_mma_takes(B, d_model, d_inner, wfmt, act));
         // x is normalised and packed once per linear (into d_gn) instead of by
-        // every block of the MFMA GEMV, whose staging is issue-bound: from 8
-        // rows (below that the extra launch costs what it saves), or from 3
-        // when both linears take the single-pass kernel with its partial sums
-        // of squares (frag_parts: one pack launch per step, not per linear;
-        // 2.7B at batch 4: 2573 against 2454 tok/s, batch 6: 3548 against 3230)
+        // every block of the staging MFMA GEMV: where gemv_rows pays; for the
+        // single-pass kernel (int4 group 64 x bf16, up to 32 rows) from 8 rows
+        // (below that the extra launch costs what it saves), or from 3 when
+        // both linears take it with its partial sums of squares (frag_parts:
+        // one pack launch per step, not per linear; 2.7B at batch 4: 2573
+        // against 2454 tok/s, batch 6: 3548 against 3230)
         const bool mmx_in = d_model % 128 == 0 && gemv_mmx_takes(B, proj, d_model, wfmt, act);
         const bool mmx_out = d_inner % 128 == 0 && gemv_mmx_takes(B, d_model, d_inner, wfmt, act);
         const uint32_t np_h = gemv_mmx_parts(B, d_model, d_inner, wfmt, act);
         const uint32_t np_g = ssd_step_parts(H, P, N, act);
         const bool parts_ok = mmx_in && mmx_out && np_h != 0 && np_g != 0;
         const uint32_t PACK_MIN_ROWS = nopack != 0 && parts_ok ? parts_min_rows : pack_min_rows;
-        const bool pack_in = B >= PACK_MIN_ROWS && d_model % 128 == 0 && gemv_mma_takes(B, proj, d_model, wfmt, act);
-        const bool pack_out = B >= PACK_MIN_ROWS && d_inner % 128 == 0 &&
-                              gemv_mma_takes(B, d_model, d_inner, wfmt, act);
-        // packed in the single-pass kernel's fragment order when it takes the call
-        const bool frag_in = pack_in && mmx_in;
-        const bool frag_out = pack_out && mmx_out;
+        // packed for the single-pass kernel, or for gemv_rows
+        const bool frag_in = B >= PACK_MIN_ROWS && mmx_in && gemv_mma_takes(B, proj, d_model, wfmt, act);
+        const bool frag_out = B >= PACK_MIN_ROWS && mmx_out && gemv_mma_takes(B, d_model, d_inner, wfmt, act);
+        const bool rows_in = !frag_in && rows_aligned && gemv_rows_pays(B, proj, d_model, wfmt, act);
+        const bool rows_out = !frag_out && rows_aligned && gemv_rows_pays(B, d_model, d_inner, wfmt, act);
+        const bool pack_in = frag_in || rows_in, pack_out = frag_out || rows_out;
+        // fused RMSNorm + linear kernels: the VALU GEMV up to 4 rows, the MFMA
+        // GEMVs for decode batches of the shapes they take
+        const bool fused_in = (B <= 4 && (int)B <= gemv_max_rows(d_model, wfmt, act)) ||
+                              (B >= 2 && gemv_mma_takes(B, proj, d_model, wfmt, act)) || rows_in;
+        const bool fused_out = (B <= 4 && gemv_max_rows(d_inner, wfmt, act) >= 1) ||
+                               (B >= 2 && gemv_mma_takes(B, d_model, d_inner, wfmt, act)) || rows_out;
         // x = r(x w) in fragment order with partial sums of squares (nopack)
         const bool frag_parts = nopack == 1 && frag_in && frag_out && parts_ok;
         const bool raw_pack = nopack == 2 && frag_in && frag_out;
@@ -346,8 +359,9 @@ struct lssm_engine {
                         // linear then rounds at the same point)
                         const bool raw = raw_pack || frag_parts;
                         e = launch_mma_pack(st(), d_hidden, d_model, w.norm_w, RMS_EPS, B, d_model, wfmt, act,
-                                            d_gn, frag_in, raw ? h_part : nullptr);
+                                            d_gn, raw ? h_part : nullptr);
                         a.g.xpack = d_gn;
+                        a.g.xrows = rows_in;
                         if (raw) {
                             a.g.xpart = h_part;
                             a.g.nparts = 4;
@@ -404,8 +418,9 @@ struct lssm_engine {
                     }
                 } else if (pack_out) {
                     e = launch_mma_pack(st(), d_g, d_inner, w.mixer_norm_w, RMS_EPS, B, d_inner, wfmt, act, d_gn,
-                                        frag_out, raw_pack ? g_part : nullptr);
+                                        raw_pack ? g_part : nullptr);
                     g.xpack = d_gn;
+                    g.xrows = rows_out;
                     if (raw_pack) {
                         g.xpart = g_part;
                         g.nparts = 4;
@@ -705,6 +720,11 @@ int lssm_engine_create(lssm_engine** out, lssm_ctx* ctx, const lssm_model_config
     e->norm_f = norm_f;
     e->lm_head = lm_head ? lm_head : embed;   // tied lm_head (mamba2_model.cpp:75-83)
     e->layers.assign(layers, layers + cfg->n_layer);
+    auto at = [](const void* p, size_t n) { return (uintptr_t)p % n == 0; };
+    e->rows_aligned = at(e->lm_head, 16) && at(norm_f, 16);
+    for (const lssm_layer_weights& w : e->layers)
+        e->rows_aligned = e->rows_aligned && at(w.norm_w, 16) && at(w.mixer_norm_w, 16) && at(w.in_proj_w, 16) &&
+                          at(w.out_proj_w, 16) && at(w.in_proj_s, 4) && at(w.out_proj_s, 4);
     e->max_batch = max_batch;
     e->max_seq = max_seq;
 

@@ -22,7 +22,8 @@
 //      int4 x bf16: nibble ^ 8 as a byte, one v_perm per pair puts it under a
 //            0x43 byte: bf16 0x43XX = 136 + q; 136 * sum(x) is subtracted per chunk;
 //      int4 x fp16: ((q ^ 8) | 0x6400) = 1032 + q, then v_pk_add_f16 -1032 (exact);
-//      int8 x fp16: ((q ^ 128) | 0x6400) = 1152 + q, then -1152 (exact).
+//      int8 x fp16: ((q ^ 128) | 0x6400) = 1152 + q, then -1152 (exact);
+//      int8 x bf16: q converted to fp32, whose upper half is q in bf16.
 //    Large N walks row groups with the next group's loads in flight
 //    (ping-pong register sets: no copies, so no early waits).
 //
@@ -871,7 +872,7 @@ template <int FMT> bool gemv1_shape(uint32_t cpr) {
 
 // Largest MR the gemv1 staging of this K / format fits (0 = not a gemv1 shape).
 inline int gemv1_rows(uint32_t K, int wfmt, int act) {
-    if (act == LSSM_F32 || (wfmt == LSSM_W_Q8_G32 && act != LSSM_F16)) return 0;
+    if (act == LSSM_F32) return 0;
     const uint32_t wpc = wpc_of(wfmt, act);
     if (K % wpc != 0) return 0;
     const uint32_t cpr = K / wpc;
@@ -1064,9 +1065,7 @@ hipError_t launch_fmt(hipStream_t s, const GemvCore& c, const Epi& e, int mr, in
             switch (wfmt) {
                 case LSSM_W_Q4_B32: err = launch_gemv1_mr<LSSM_W_Q4_B32, T, Epi>(s, c, e, mr, norm, done); break;
                 case LSSM_W_Q4_G64: err = launch_gemv1_mr<LSSM_W_Q4_G64, T, Epi>(s, c, e, mr, norm, done); break;
-                case LSSM_W_Q8_G32:
-                    if constexpr (__is_same(T, f16)) err = launch_gemv1_mr<LSSM_W_Q8_G32, T, Epi>(s, c, e, mr, norm, done);
-                    break;
+                case LSSM_W_Q8_G32: err = launch_gemv1_mr<LSSM_W_Q8_G32, T, Epi>(s, c, e, mr, norm, done); break;
                 default: err = launch_gemv1_mr<LSSM_W_DENSE, T, Epi>(s, c, e, mr, norm, done); break;
             }
             if (done) return err;
@@ -1165,6 +1164,7 @@ __global__ void dequant_kernel(const uint8_t* __restrict__ w, const uint16_t* __
 }  // namespace
 
 int gemv_max_rows(uint32_t K, int wfmt, int act) { return max_rows(K, wfmt, act); }
+bool gemv1_takes(uint32_t K, int wfmt, int act) { return gemv1_rows(K, wfmt, act) > 0; }
 
 hipError_t launch_gemv_argmax(hipStream_t s, const GemvArgs& a, int32_t* ids, void* scratch,
                               size_t scratch_bytes) {

@@ -355,6 +355,17 @@ __device__ __forceinline__ Unpacked<FMT, T> unpack(const uint4 wv) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) u.p[4 * i + j] = pk_add_f16(((v >> (4 * j)) & 0x000F000Fu) | 0x64006400u, -1032.0f);
         }
+    } else if constexpr (FMT == LSSM_W_Q8_G32 && __is_same(T, bf16)) {
+        // q as fp32 is exact in its upper 16 bits, which are its bf16 (|q| <=
+        // 128: 8 significand bits); v_perm takes the upper halves of two
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t f[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[e] = __float_as_uint((float)(int8_t)(d[i] >> (8 * e)));
+            u.p[2 * i] = __builtin_amdgcn_perm(f[2], f[0], 0x07060302u);
+            u.p[2 * i + 1] = __builtin_amdgcn_perm(f[3], f[1], 0x07060302u);
+        }
     } else if constexpr (FMT == LSSM_W_Q8_G32) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {

@@ -4,7 +4,7 @@
 #include <algorithm>
 #include <cstdlib>
 
-#include "gemv_core.hpp"
+#include "gemv_mma_core.hpp"
 
 namespace lssm {
 
@@ -47,107 +47,10 @@ constexpr bool mma_shape_ok(int ct, int qpw, bool q4) {
            (q4 && ((qpw == 2 && ct >= 2 && ct <= 4) || (ct == 4 && qpw == 4)));
 }
 constexpr int MM_MAXJ = 8;                       // staged octets per thread and pass
-constexpr size_t MM_LDS_MAX = 150 * 1024;        // dynamic LDS (static: < 5 KiB)
-
-template <int V> struct FmtTag {
-    static constexpr int value = V;
-};
-
-template <int FMT, typename T> struct Mma {
-    using F = Fmt<FMT, T>;
-    static constexpr int WPC = F::WPC;
-    static constexpr int NP = WPC / 2;                                  // pairs per chunk
-    static constexpr int QK = 4 * WPC;                                  // k per quad
-    static constexpr int G = F::G;                                      // 0: dense
-    static constexpr int SPQ = FMT == LSSM_W_DENSE ? 1 : (FMT == LSSM_W_Q8_G32 ? 2 : 4);  // MFMAs per quad
-    static constexpr int GPQ = G ? QK / G : 1;                          // scale groups per quad
-    static constexpr int SPG = SPQ / GPQ;                               // MFMAs per group
-    static constexpr bool BIAS = q4_bf16<FMT, T>();
-};
-
-// Chunk (within the quad) and pair offset of MFMA k-slice s of lane group q,
-// after mma_swap: the x pairs that slice s meets in lane group q.
-template <int FMT> __device__ __forceinline__ void mma_slice_pos(int s, int q, int& ch, int& po) {
-    if constexpr (FMT == LSSM_W_Q4_G64) {
-        ch = (q & 1) + 2 * (s >> 1);
-        po = 4 * ((s & 1) + 2 * (q >> 1));
-    } else if constexpr (FMT == LSSM_W_Q4_B32) {
-        ch = s;
-        po = 4 * q;
-    } else if constexpr (FMT == LSSM_W_Q8_G32) {
-        ch = (q & 1) + 2 * s;
-        po = 4 * (q >> 1);
-    } else {
-        ch = q;
-        po = 0;
-    }
-}
-
-// Lane group q loaded chunk q of the quad (dwords C_q[0..3]).  After the
-// 32-lane swap, lane group q holds C_{q&1}[2(q>>1)], C_{q&1}[2(q>>1)+1],
-// C_{(q&1)+2}[2(q>>1)], C_{(q&1)+2}[2(q>>1)+1]: dwords 0-1 come from chunks
-// 0-1 and dwords 2-3 from chunks 2-3 (one 64-wide group each).  After the
-// 16-lane swap as well it holds C_0[q], C_1[q], C_2[q], C_3[q] (dword j from
-// chunk j: one 32-wide group each).
-template <int FMT> __device__ __forceinline__ u32x4 mma_swap(u32x4 v) {
-    if constexpr (FMT == LSSM_W_DENSE) {
-        return v;
-    } else {
-        const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
-        const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
-        u32x4 r = u32x4{a[0], b[0], a[1], b[1]};
-        if constexpr (FMT == LSSM_W_Q4_B32) {
-            const auto c = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
-            const auto d = __builtin_amdgcn_permlane16_swap(r[2], r[3], false, false);
-            r = u32x4{c[0], c[1], d[0], d[1]};
-        }
-        return r;
-    }
-}
-
-// Pair q of an octet (8 consecutive k, 8-aligned) in pair_pos order: the
-// positions (within the octet) of its two values.  Octets never straddle the
-// pair structure of a chunk, so these are constants.
-template <int FMT, typename T> __device__ __forceinline__ void octet_pos(int q, int& a, int& b) {
-    if constexpr (q4_bf16<FMT, T>()) {
-        a = ((q & 2) ? 1 : 0) + ((q & 1) ? 4 : 0);
-        b = a + 2;
-    } else if constexpr (is_q4<FMT>()) {
-        a = q;
-        b = q + 4;
-    } else if constexpr (FMT == LSSM_W_Q8_G32) {
-        a = 4 * (q / 2) + q % 2;
-        b = a + 2;
-    } else {
-        a = 2 * q;
-        b = a + 1;
-    }
-}
-
-// The 8 weights of MFMA k-slice s of a swapped quad as packed pairs: dword s
-// (int4), dwords 2s, 2s+1 (int8), the whole quad chunk (dense).
-template <int FMT, typename T> __device__ __forceinline__ u32x4 unpack_slice(u32x4 v, int s) {
-    if constexpr (FMT == LSSM_W_DENSE) {
-        return v;
-    } else if constexpr (FMT == LSSM_W_Q8_G32) {
-        const Unpacked<FMT, T> u = unpack<FMT, T>(make_uint4(v[2 * s], v[2 * s + 1], 0u, 0u));
-        return u32x4{u.p[0], u.p[1], u.p[2], u.p[3]};
-    } else {
-        const Unpacked<FMT, T> u = unpack<FMT, T>(make_uint4(v[s], 0u, 0u, 0u));
-        return u32x4{u.p[0], u.p[1], u.p[2], u.p[3]};
-    }
-}
-
-template <typename T> __device__ __forceinline__ floatx4 mfma16(u32x4 a, u32x4 b, floatx4 c) {
-    if constexpr (__is_same(T, bf16))
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
-}
 
 // ra: dwords of the LDS region that holds, in turn, the lanes' sums of
 // squares, the staged x rows and each pass's partial sums.
-template <int FMT, typename T, int CT, int QPW, bool NORM, bool PACKED, class Epi>
+template <int FMT, typename T, int CT, int QPW, bool NORM, class Epi>
 __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvCore c, Epi epi, uint32_t M, uint32_t mpb,
                                                                  uint32_t ra) {
     using P = Mma<FMT, T>;
@@ -304,34 +207,6 @@ __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvC
         lds_barrier();
     };
 
-    // ---- x pre-packed by launch_mma_pack: rows [base, base + mpb) copied ----
-    // (16-byte pieces p = row * KO + octet, eight in flight per thread)
-    auto copy_in = [&](uint32_t base) {
-        const uint32_t NT = blockDim.x, KH = K / 2;
-        const uint32_t n = min(mpb, M - base) * KO;
-        const uint32_t ko_magic = 0xFFFFFFFFu / KO + 1u;           // KO >= 16: exact for p < 2^16
-        for (uint32_t p0 = threadIdx.x; p0 < n; p0 += 8 * NT) {
-            u32x4 v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint32_t p = p0 + i * NT;
-                if (p < n) {
-                    const uint32_t r = __umulhi(p, ko_magic), cc = p - r * KO;
-                    v[i] = *reinterpret_cast<const u32x4*>(c.xp + (size_t)(base + r) * KH + 4 * cc);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint32_t p = p0 + i * NT;
-                if (p < n) {
-                    const uint32_t r = __umulhi(p, ko_magic), cc = p - r * KO;
-                    *reinterpret_cast<u32x4*>(xl + r * RS + 4 * cc) = v[i];
-                }
-            }
-        }
-        lds_barrier();
-    };
-
     // ---- weights (and raw scale bits) of the wave's quads, all in flight ----
     // With few weight registers (CT * QPW <= 8) they are held over all
     // passes; otherwise a later pass reads them again (L2 hits) rather than
@@ -375,8 +250,7 @@ __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvC
     // x of the first pass, staged before any weight is requested: requested
     // behind the weights, x would queue behind the whole chip's weight
     // traffic (measured: staging done ~7 us after the start instead of ~2)
-    constexpr bool packed = PACKED;                            // x from launch_mma_pack (c.xp)
-    const bool keep0 = !packed && mpb * SEG <= (uint32_t)(MM_MAXJ * KS);   // the first pass's x fits the registers
+    const bool keep0 = mpb * SEG <= (uint32_t)(MM_MAXJ * KS);   // the first pass's x fits the registers
     if (keep0) {
         const uint32_t nseg = mpb * SEG;
         const uint32_t lane0 = threadIdx.x % WAVE;
@@ -396,15 +270,13 @@ __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvC
             }
         }
     }
-    if (packed) copy_in(0u);
-    else if (keep0) stage(0u, FmtTag<1>{});
+    if (keep0) stage(0u, FmtTag<1>{});
     else stage(0u, FmtTag<0>{});
     load_w();
 
     for (uint32_t base = 0; base < M; base += mpb) {
         if (base > 0) {
-            if (packed) copy_in(base);
-            else stage(base, FmtTag<0>{});
+            stage(base, FmtTag<0>{});
             if constexpr (!HOLD) load_w();
         }
         const uint32_t rows = min(mpb, M - base);
@@ -1199,9 +1071,9 @@ template <typename T> bool mma_aligned(const GemvCore& c, bool norm) {
            (!norm || (uintptr_t)c.norm_w % 16 == 0) && (uintptr_t)c.w % 16 == 0 && (uintptr_t)c.s % 16 == 0;
 }
 
-template <int FMT, typename T, int CT, int QPW, bool NORM, bool PACKED, class Epi>
+template <int FMT, typename T, int CT, int QPW, bool NORM, class Epi>
 hipError_t mma_run(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, const MmaPlan& p) {
-    auto k = gemv_mma_kernel<FMT, T, CT, QPW, NORM, PACKED, Epi>;
+    auto k = gemv_mma_kernel<FMT, T, CT, QPW, NORM, Epi>;
     // opt in to the dynamic LDS once per instantiation (a host attribute)
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MM_LDS_MAX);
@@ -1211,22 +1083,22 @@ hipError_t mma_run(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, c
     return hipGetLastError();
 }
 
-template <int FMT, typename T, bool NORM, bool PACKED, class Epi>
+template <int FMT, typename T, bool NORM, class Epi>
 hipError_t mma_shape(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, const MmaPlan& p) {
     if (p.ct == 1) {
         switch (p.qpw) {
-            case 1: return mma_run<FMT, T, 1, 1, NORM, PACKED, Epi>(s, c, e, M, p);
-            case 2: return mma_run<FMT, T, 1, 2, NORM, PACKED, Epi>(s, c, e, M, p);
-            case 4: return mma_run<FMT, T, 1, 4, NORM, PACKED, Epi>(s, c, e, M, p);
-            default: return mma_run<FMT, T, 1, 8, NORM, PACKED, Epi>(s, c, e, M, p);
+            case 1: return mma_run<FMT, T, 1, 1, NORM, Epi>(s, c, e, M, p);
+            case 2: return mma_run<FMT, T, 1, 2, NORM, Epi>(s, c, e, M, p);
+            case 4: return mma_run<FMT, T, 1, 4, NORM, Epi>(s, c, e, M, p);
+            default: return mma_run<FMT, T, 1, 8, NORM, Epi>(s, c, e, M, p);
         }
     }
     if constexpr (FMT == LSSM_W_Q4_G64 || FMT == LSSM_W_Q4_B32) {
-        if (p.qpw == 4) return mma_run<FMT, T, 4, 4, NORM, PACKED, Epi>(s, c, e, M, p);
+        if (p.qpw == 4) return mma_run<FMT, T, 4, 4, NORM, Epi>(s, c, e, M, p);
         switch (p.ct) {
-            case 2: return mma_run<FMT, T, 2, 2, NORM, PACKED, Epi>(s, c, e, M, p);
-            case 3: return mma_run<FMT, T, 3, 2, NORM, PACKED, Epi>(s, c, e, M, p);
-            default: return mma_run<FMT, T, 4, 2, NORM, PACKED, Epi>(s, c, e, M, p);
+            case 2: return mma_run<FMT, T, 2, 2, NORM, Epi>(s, c, e, M, p);
+            case 3: return mma_run<FMT, T, 3, 2, NORM, Epi>(s, c, e, M, p);
+            default: return mma_run<FMT, T, 4, 2, NORM, Epi>(s, c, e, M, p);
         }
     }
     return hipErrorInvalidValue;                       // not a planned shape
@@ -1280,12 +1152,11 @@ bool try_mma(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, int wfm
             err = mmx_go<FMT, T, Epi>(s, c, e, M, q);
             return true;
         }
-        if (c.part) {                                          // raw x: only the single-pass kernel
+        if (c.xp) {                                            // packed x: only the single-pass kernel
             err = hipErrorInvalidValue;
             return true;
         }
-        err = c.xp ? mma_shape<FMT, T, true, true, Epi>(s, c, e, M, p)
-                   : mma_shape<FMT, T, true, false, Epi>(s, c, e, M, p);
+        err = mma_shape<FMT, T, true, Epi>(s, c, e, M, p);
         return true;
     });
 }
@@ -1298,24 +1169,22 @@ template <typename T> bool mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfm
     });
 }
 
-// ---- x normalised and packed once for a whole gemv_mma launch ----
+// ---- x normalised and packed once for a whole launch ----
 // Row m: rr = 1 / sqrt(mean(x^2) + eps), then each octet's r(x w rr) in the
-// staging's pair order (norm.metal:52-79), stored as the staging would put it
-// in LDS (pairs of k .. k + 7 at dwords k / 2 .. k / 2 + 3 of the row) or, with
-// FRAG (int4 group 64 only), in gemv_mmx_kernel's fragment order: the 16 bytes
-// lane l = 16 q + (m % 16) supplies to k-slice s of quad qa for row tile m / 16
-// at u32x4 ((m / 16 quads + qa) 4 + s) 64 + l.  With FRAG the grid covers the
-// rows up to the next multiple of 16, and rows past M are zeros.
-template <int FMT, typename T, bool FRAG>
+// unpack's pair order (norm.metal:52-79), stored in the fragment order of
+// gemv_mmx_kernel and gemv_rows_kernel: the 16 bytes lane l = 16 q + (m % 16)
+// supplies to k-slice s of quad qa for row tile m / 16 at u32x4 ((m / 16 quads
+// + qa) SPQ + s) 64 + l.  The grid covers the rows up to the next multiple of
+// 16; rows past M are zeros.
+template <int FMT, typename T>
 __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_stride, const T* nw, float eps,
                                                         uint32_t K, uint32_t M, uint32_t* out, float* part) {
     // one octet per thread (blockDim.x >= K / 8), x and w read once
     __shared__ float red[1024 / WAVE];
     const uint32_t m = blockIdx.x, KO = K / 8, cc = threadIdx.x;
     const bool live = cc < KO;
-    const bool row = !FRAG || m < M;
     u32x4 xv = u32x4{0u, 0u, 0u, 0u}, nv = xv;
-    if (live && row) {
+    if (live && m < M) {
         xv = reinterpret_cast<const u32x4*>(x + (size_t)m * x_stride)[cc];
         nv = reinterpret_cast<const u32x4*>(nw)[cc];
     }
@@ -1332,7 +1201,7 @@ __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_s
     for (uint32_t i = 0; i < nwv; ++i) t += red[i];
     const float rr = 1.0f / sqrtf(t / (float)K + eps);
     // part: x w without 1 / rms, the sum of squares to part[4 m]
-    const bool raw = FRAG && part != nullptr;
+    const bool raw = part != nullptr;
     if (raw && threadIdx.x < 4) part[4 * m + threadIdx.x] = threadIdx.x == 0 ? t : 0.0f;
     if (!live) return;
     const float sc = raw ? 1.0f : rr;
@@ -1349,42 +1218,37 @@ __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_s
         octet_pos<FMT, T>(qq, pa, pb);
         pk[qq] = pack2<T>(v[pa], v[pb]);
     }
-    if constexpr (FRAG) {
-        // octet cc = 16 qa + 4 ch + p (chunk ch, pair offset 4 p of the quad):
-        // k-slice s and lane group q with mma_slice_pos(s, q) = (ch, 4 p)
-        const uint32_t qa = cc / 16, ch = (cc % 16) / 4, p4 = cc % 4;
-        const uint32_t sl = 2 * (ch >> 1) + (p4 & 1), lg = (ch & 1) + 2 * (p4 >> 1);
-        const uint32_t quads = K / 128;
-        reinterpret_cast<u32x4*>(out)[(((size_t)(m / 16) * quads + qa) * 4 + sl) * WAVE + 16 * lg + m % 16] = pk;
-    } else {
-        reinterpret_cast<u32x4*>(out + (size_t)m * (K / 2))[cc] = pk;
-    }
+    // octet cc of quad qa: chunk ch, pair offset 4 p4 of the chunk; k-slice sl
+    // and lane group lg with mma_slice_pos(sl, lg) = (ch, 4 p4)
+    using P = Mma<FMT, T>;
+    constexpr uint32_t OPQ = P::QK / 8, OPC = OPQ / 4;             // octets per quad, per chunk
+    const uint32_t qa = cc / OPQ, ch = (cc % OPQ) / OPC, p4 = cc % OPC;
+    uint32_t sl, lg;
+    if constexpr (FMT == LSSM_W_Q4_G64) sl = 2 * (ch >> 1) + (p4 & 1), lg = (ch & 1) + 2 * (p4 >> 1);
+    else if constexpr (FMT == LSSM_W_Q4_B32) sl = ch, lg = p4;
+    else if constexpr (FMT == LSSM_W_Q8_G32) sl = ch >> 1, lg = (ch & 1) + 2 * p4;
+    else sl = 0, lg = ch;
+    const uint32_t quads = K / P::QK;
+    reinterpret_cast<u32x4*>(out)[(((size_t)(m / 16) * quads + qa) * P::SPQ + sl) * WAVE + 16 * lg + m % 16] = pk;
 }
 
 }  // namespace
 
 hipError_t launch_mma_pack(hipStream_t s, const void* x, uint32_t x_stride, const void* norm_w, float eps,
-                           uint32_t M, uint32_t K, int wfmt, int act, void* out, bool frag, float* part) {
-    if (M == 0 || K % 128 != 0 || K > 8192 || (uintptr_t)x % 16 || (x_stride * 2u) % 16 ||
-        (uintptr_t)norm_w % 16 || (uintptr_t)out % 16)
+                           uint32_t M, uint32_t K, int wfmt, int act, void* out, float* part) {
+    if (M == 0 || K > 8192 || (uintptr_t)x % 16 || (x_stride * 2u) % 16 || (uintptr_t)norm_w % 16 || (uintptr_t)out % 16)
         return hipErrorInvalidValue;
-    if (frag && (wfmt != LSSM_W_Q4_G64 || act != LSSM_BF16)) return hipErrorInvalidValue;
-    if (part && !frag) return hipErrorInvalidValue;
+    if (part && (wfmt != LSSM_W_Q4_G64 || act != LSSM_BF16)) return hipErrorInvalidValue;
     const uint32_t nt = (K / 8 + WAVE - 1) / WAVE * WAVE;      // one octet per thread
-    if (frag) {
-        mma_pack_kernel<LSSM_W_Q4_G64, bf16, true><<<(M + 15) / 16 * 16, nt, 0, s>>>(
-            static_cast<const bf16*>(x), x_stride, static_cast<const bf16*>(norm_w), eps, K, M,
-            static_cast<uint32_t*>(out), part);
-        return hipGetLastError();
-    }
     hipError_t err = hipErrorInvalidValue;
     auto go = [&](auto tag) -> bool {
         using T = decltype(tag);
-        return mma_fmt<T>(wfmt, [&](auto ft) -> bool {
+        return all_fmt<T>(wfmt, [&](auto ft) -> bool {
             constexpr int FMT = decltype(ft)::value;
-            mma_pack_kernel<FMT, T, false><<<M, nt, 0, s>>>(static_cast<const T*>(x), x_stride,
-                                                             static_cast<const T*>(norm_w), eps, K, M,
-                                                             static_cast<uint32_t*>(out), nullptr);
+            if (K % Mma<FMT, T>::QK != 0) return false;
+            mma_pack_kernel<FMT, T><<<(M + 15) / 16 * 16, nt, 0, s>>>(
+                static_cast<const T*>(x), x_stride, static_cast<const T*>(norm_w), eps, K, M,
+                static_cast<uint32_t*>(out), part);
             err = hipGetLastError();
             return true;
         });
@@ -1408,6 +1272,23 @@ uint32_t gemv_mmx_parts(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) {
     return N % 128 == 0 && np % 4 == 0 && np <= MMX_MAXPARTS ? np : 0;
 }
 
+uint64_t gemv_mma_staged(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) {
+    uint64_t v = 0;
+    auto plan = [&](auto tag) {
+        using T = decltype(tag);
+        mma_fmt<T>(wfmt, [&](auto ft) -> bool {
+            MmaPlan p;
+            if (M < mma_min_rows() || !mma_plan<decltype(ft)::value, T>(M, N, K, p) || p.mpb < M) return false;
+            const uint32_t blocks = ((N + 15) / 16 + p.ct - 1) / p.ct;
+            v = (uint64_t)((blocks + num_cus() - 1) / num_cus()) * M * K;
+            return true;
+        });
+    };
+    if (act == LSSM_F16) plan(f16{});
+    else if (act == LSSM_BF16) plan(bf16{});
+    return v;
+}
+
 bool gemv_mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) {
     if (act == LSSM_F16) return mma_takes<f16>(M, N, K, wfmt);
     if (act == LSSM_BF16) return mma_takes<bf16>(M, N, K, wfmt);
@@ -1415,6 +1296,7 @@ bool gemv_mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) {
 }
 
 bool launch_gemv_mma(hipStream_t s, const GemvArgs& a, hipError_t& err) {
+    if (a.xrows) return launch_gemv_rows(s, a, err);
     if (a.M < 2 && !a.yfrag) return false;
     GemvCore c{a.x, a.x_stride, (const uint8_t*)a.w, (const uint16_t*)a.s, a.norm_w, a.eps, a.N, a.K, 1.0f / (float)a.K};
     c.xp = static_cast<const uint32_t*>(a.xpack);
@@ -1477,6 +1359,7 @@ bool launch_inproj_ssd_decode_mma(hipStream_t s, const InprojDecodeArgs& a, cons
 
 bool launch_inproj_decode_mma(hipStream_t s, const InprojDecodeArgs& a, hipError_t& err) {
     const GemvArgs& g = a.g;
+    if (g.xrows) return launch_inproj_rows(s, a, err);
     if (g.M < 2) return false;
     GemvCore c{g.x, g.x_stride, (const uint8_t*)g.w, (const uint16_t*)g.s, g.norm_w, g.eps, g.N, g.K, 1.0f / (float)g.K};
     c.xp = static_cast<const uint32_t*>(g.xpack);

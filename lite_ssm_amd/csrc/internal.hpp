@@ -36,6 +36,8 @@ struct lssm_ctx {
     float* ssd_gram = nullptr;
     size_t ssd_gram_cap = 0;   // floats
     std::vector<float*> ssd_gram_retired;
+    // x rows packed for the batched decode GEMV (lssm::GEMV_PACK_BYTES)
+    void* xpack = nullptr;
 };
 
 namespace lssm {
@@ -144,6 +146,8 @@ struct GemvArgs {
     // x rows as launch_mma_pack wrote them (norm_w applied), or null; used by
     // the MFMA decode GEMV, which then copies instead of normalising
     const void* xpack = nullptr;
+    // xpack is for the gemv_rows kernel, which takes the call (gemv_rows_takes)
+    bool xrows = false;
     // with xpack in fragment order: xpack holds r(x norm_w) without the
     // rows' 1 / rms, which the GEMV forms from their partial sums of squares
     // of x ([rows][nparts], added in order) and applies to its fp32 sums;
@@ -386,20 +390,42 @@ bool launch_inproj_ssd_decode_mma(hipStream_t s, const InprojDecodeArgs& a, cons
 // Whether a decode batch of M rows runs in one MFMA launch (16-byte aligned
 // operands assumed; otherwise the launchers fall back to gemv1 launches).
 bool gemv_mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
-// RMSNorm of M rows of x (K, 16-bit act), rounded and packed in the MFMA
-// decode GEMV's staging order for `wfmt`, into out ([M][K / 2] dwords): one
-// pass for all blocks of the GEMV launch that follows (GemvArgs::xpack).
+// RMSNorm of M rows of x (K <= 8192, 16-bit act), rounded and packed in the
+// fragment order of the single-pass MFMA GEMV and of gemv_rows for `wfmt`, into
+// out (ceil(M / 16) * 16 rows of K): one pass for all blocks of the GEMV
+// launch that follows (GemvArgs::xpack).
+// With part set (int4 group 64 x bf16), the rows are written as r(x norm_w),
+// without 1 / rms, and row m's sum of squares goes to part[4 m], zeros to
+// part[4 m + 1 .. 4 m + 3]: four partials a row, for the GEMV that scales its
+// sums by 1 / rms (GemvArgs::xpart); rows up to ceil(M / 16) * 16.
 hipError_t launch_mma_pack(hipStream_t s, const void* x, uint32_t x_stride, const void* norm_w,
                            float eps, uint32_t M, uint32_t K, int wfmt, int act, void* out,
-                           bool frag = false, float* part = nullptr);
-// (with frag and part set, the rows are written as r(x norm_w), without
-// 1 / rms, and row m's sum of squares goes to part[4 m], zeros to part[4 m +
-// 1 .. 4 m + 3]: four partials a row, for the GEMV that scales its sums by
-// 1 / rms (GemvArgs::xpart); rows up to ceil(M / 16) * 16)
+                           float* part = nullptr);
 // The MFMA decode GEMV takes (M, N, K) in its single-pass form, which reads x
-// packed in fragment order (launch_mma_pack with frag = true; the buffer then
-// holds ceil(M / 16) * 16 rows).
+// packed in fragment order (launch_mma_pack).
 bool gemv_mmx_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
+// The decode GEMV for any 16-bit activation type and weight format (gemv_rows)
+// takes (M, N, K): 1..64 rows, K of whole quads (int4 128, int8 64, dense 32)
+// and at most 8192; x packed by launch_mma_pack.
+bool gemv_rows_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
+// Dense weights of so many rows (the lm_head) that the tiled GEMM behind a norm
+// launch streams them faster, past four rows of x: it reads them in runs of
+// 128 bytes a row, a tile's rows at a time (50280 x 2560 at 16 rows: 57.6
+// against 68 us; at K below 2048 gemv_rows is ahead: 50280 x 768 15 against
+// 20.9).
+bool dense_head_gemm(uint32_t N, uint32_t K, int wfmt, int act);
+// Whether packing x and running it is the fastest way to take a decode linear
+// of M rows with its RMSNorm.
+bool gemv_rows_pays(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
+// x values the staging MFMA kernel (launch_gemv_mma without xpack) stages per
+// CU for this call when one pass takes all rows; 0 where it does not.
+uint64_t gemv_mma_staged(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
+// Whether the VALU GEMV of up to four rows (gemv1) has this K and format.
+bool gemv1_takes(uint32_t K, int wfmt, int act);
+bool launch_gemv_rows(hipStream_t s, const GemvArgs& a, hipError_t& err);
+bool launch_inproj_rows(hipStream_t s, const InprojDecodeArgs& a, hipError_t& err);
+// Bytes of x packed for it, at most.
+constexpr size_t GEMV_PACK_BYTES = (size_t)64 * 8192 * 2;
 // Partials per row (N / 16) the single-pass MFMA GEMV writes for (M, N, K)
 // with GemvArgs::yfrag, or 0 when it cannot (another plan, or a count the
 // GEMV that reads them does not take).

@@ -61,3 +61,68 @@ def test_fp32_gemm_dense_short_k_strides_epilogues(ctx, rng, M, N, K):
         ctx.linear(dev(x), dev(w), _sdev(s), y2, M, N, K, wfmt, O.F32, epi=L.EPI_SILU)
         ref = O.linear(O.to_act(x, O.F32), w, s, M, N, K, wfmt, O.F32, epi=O.EPI_SILU, round_dequant=1)
         assert_close(act_host(y2, O.F32), ref, O.F32, 1e-5, "silu")
+
+
+# --------------------------------------------------------------------------- batched decode GEMV
+def _norm_linear(ctx, x, nw, w, s, M, N, K, wfmt, act, res=None):
+    import lite_ssm_amd as L
+    y = dev(res) if res is not None else empty((M, N), act)
+    L.check(L.lib.lssm_norm_linear_decode(ctx.h, dev(x).data_ptr(), dev(nw).data_ptr(), 1e-5, dev(w).data_ptr(),
+                                          None if s is None else dev(s).data_ptr(), y.data_ptr(),
+                                          y.data_ptr() if res is not None else None, M, N, K, wfmt, act,
+                                          L.EPI_NONE if res is None else L.EPI_ADD))
+    return act_host(y, act)
+
+
+# Rows at the edges of the 16-row tiles; widths for 1, 2, 3, 4 and 5 tiles of W
+# per block and for more tiles than five per CU, with a partial last tile;
+# depths of one quad (seven waves idle), ten (an uneven split) and the most;
+# and a dense weight wide enough for the tiled GEMM behind a norm launch.
+@pytest.mark.parametrize("act", [O.F16, O.BF16])
+@pytest.mark.parametrize("wfmt", ALL_FMTS)
+@pytest.mark.parametrize("N,K", [(40, 128), (300, 1280), (72, 8192), (5000, 256), (9001, 128), (13000, 256),
+                                 (17000, 256), (25000, 128), (32780, 2048)])
+def test_decode_rows_vs_oracle(ctx, rng, act, wfmt, N, K):
+    if N > 32768 and wfmt != O.W_DENSE:
+        pytest.skip("dense only")
+    import lite_ssm_amd as L
+    nw = O.to_act(1 + 0.1 * rng.standard_normal(K), act)
+    w, s = _weights(rng, N, K, wfmt, act)
+    for M in (5, 16, 17, 33, 64):
+        print(f"case: decode rows act {act} fmt {wfmt} {M} x {N} x {K}", flush=True)
+        x = O.to_act(rng.standard_normal((M, K)), act)
+        res = O.to_act(rng.standard_normal((M, N)), act) if M == 17 else None
+        got = _norm_linear(ctx, x, nw, w, s, M, N, K, wfmt, act, res)
+        xn = O.rmsnorm(x, nw, 1e-5, act)
+        ref = O.linear(xn, w, s, M, N, K, wfmt, act, epi=O.EPI_NONE if res is None else O.EPI_ADD, residual=res)
+        assert_close(got, ref, act, {O.F16: 2e-3, O.BF16: 1.6e-2}[act], "decode rows")
+
+
+@pytest.mark.parametrize("act", [O.F16, O.BF16])
+@pytest.mark.parametrize("M", [1, 2, 4])
+def test_decode_rows_few_dense_deep(ctx, rng, act, M):
+    """One to four rows of a dense weight too deep for the VALU GEMV's table."""
+    N, K = 72, 8192
+    nw = O.to_act(1 + 0.1 * rng.standard_normal(K), act)
+    w, s = _weights(rng, N, K, O.W_DENSE, act)
+    x = O.to_act(rng.standard_normal((M, K)), act)
+    print(f"case: decode rows dense act {act} {M} x {N} x {K}", flush=True)
+    got = _norm_linear(ctx, x, nw, w, s, M, N, K, O.W_DENSE, act)
+    ref = O.linear(O.rmsnorm(x, nw, 1e-5, act), w, s, M, N, K, O.W_DENSE, act)
+    assert_close(got, ref, act, {O.F16: 2e-3, O.BF16: 1.6e-2}[act], "decode rows")
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("K", [768, 1536, 2560])
+def test_gemv_int8_bf16(ctx, rng, M, K):
+    """int8 weights against bf16 rows in the VALU GEMV (every int8 value is a
+    bf16), the extreme values among them."""
+    N, act = 200, O.BF16
+    x = O.to_act(rng.standard_normal((M, K)), act)
+    w, s = _weights(rng, N, K, O.W_Q8_G32, act)
+    w.view(np.int8).reshape(-1)[:256] = np.arange(-128, 128)
+    y = empty((M, N), act)
+    print(f"case: int8 x bf16 GEMV {M} x {N} x {K}", flush=True)
+    ctx.linear(dev(x), dev(w), dev(s), y, M, N, K, O.W_Q8_G32, act)
+    ref = O.linear(x, w, s, M, N, K, O.W_Q8_G32, act)
+    assert_close(act_host(y, act), ref, act, 1.6e-2, "gemv")
