@@ -80,7 +80,23 @@ int linear_core(lssm_ctx* ctx, const void* x, uint32_t xs, const void* w, const 
         e = launch_gemv(ctx->stream, g);
     } else if (!gemv && gemm_ok(x, xs, w, K, act)) {
         GemmArgs g{x, xs, w, s, y, ys, res, M, N, K, wfmt, act, epi, 1};
-        e = launch_gemm(ctx->stream, g);
+        std::unique_lock<std::mutex> lk(ctx->scratch_mu, std::defer_lock);
+        const bool split = gemm_wants_ws(g);
+        if (split) lk.lock();
+        if (split && !ctx->gemm_ws) {
+            // (not while the stream is captured: the call then runs unsplit)
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+                hipMalloc((void**)&ctx->gemm_ws, GEMM_WS_FLOATS * sizeof(float)) != hipSuccess) {
+                ctx->gemm_ws = nullptr;
+                (void)hipGetLastError();
+            }
+        }
+        if (split && ctx->gemm_ws) {
+            g.ws = ctx->gemm_ws;
+            g.ws_floats = GEMM_WS_FLOATS;
+        }
+        e = launch_gemm(ctx->stream, g);   // (the lock ends with this block, before finish() waits)
     } else {
         GemmArgs g{x, xs, w, s, y, ys, res, M, N, K, wfmt, act, epi, gemv ? 0 : 1};
         e = launch_gemm_simple(ctx->stream, g);
@@ -138,6 +154,7 @@ int lssm_norm_linear_decode(lssm_ctx* ctx, const void* x, const void* norm_w, fl
     LSSM_REQUIRE(gemv_ok(w, K, wfmt, act), "norm_linear_decode: unsupported K / weight alignment");
     GemvArgs g{x, K, w, w_scales, y, N, residual, norm_w, eps, rows, N, K, wfmt, act, epi};
     hipError_t e;
+    std::unique_lock<std::mutex> lk(ctx->scratch_mu);
     if (rows > 4 && dense_head_gemm(N, K, wfmt, act) && al16(x) && al16(norm_w)) {
         // an lm_head: norm launch, then the tiled GEMM (dense: one rule)
         e = launch_rmsnorm(ctx->stream, x, K, norm_w, ctx->xpack, K, rows, K, eps, act);
@@ -147,6 +164,7 @@ int lssm_norm_linear_decode(lssm_ctx* ctx, const void* x, const void* norm_w, fl
         e = pack_rows_ok(ctx, g) ? pack_rows(ctx, g) : hipSuccess;
         if (e == hipSuccess) e = launch_gemv(ctx->stream, g);
     }
+    lk.unlock();
     if (e != hipSuccess) return set_error(LSSM_EDEVICE, "norm_linear_decode: %s", hipGetErrorString(e));
     return finish(ctx, "norm_linear_decode");
 }
@@ -337,8 +355,12 @@ int lssm_inproj_decode(lssm_ctx* ctx, const void* hidden, const void* norm_w, co
     a.z = z;
     a.xbc_act = xbc_act;
     a.dt = dt;
-    hipError_t e = pack_rows_ok(ctx, a.g) ? pack_rows(ctx, a.g) : hipSuccess;
-    if (e == hipSuccess) e = launch_inproj_decode(ctx->stream, a);
+    hipError_t e = hipSuccess;
+    {
+        std::lock_guard<std::mutex> lk(ctx->scratch_mu);
+        if (pack_rows_ok(ctx, a.g)) e = pack_rows(ctx, a.g);
+        if (e == hipSuccess) e = launch_inproj_decode(ctx->stream, a);
+    }
     if (e != hipSuccess) return set_error(LSSM_EDEVICE, "inproj_decode: %s", hipGetErrorString(e));
     return finish(ctx, "inproj_decode");
 }

@@ -135,6 +135,7 @@ int lssm_ctx_destroy(lssm_ctx* ctx) {
     (void)hipFree(ctx->status);
     (void)hipFree(ctx->xpack);
     (void)hipHostFree(ctx->status_host);
+    if (ctx->gemm_ws) (void)hipFree(ctx->gemm_ws);
     if (ctx->ssd_seg) (void)hipFree(ctx->ssd_seg);
     if (ctx->ssd_gram) (void)hipFree(ctx->ssd_gram);
     for (float* p : ctx->ssd_gram_retired) (void)hipFree(p);

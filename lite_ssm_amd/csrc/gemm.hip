@@ -12,28 +12,13 @@
 // padded to 72 elements so the 16-byte fragment reads of 8 consecutive rows
 // hit distinct banks); the global loads of step k+1 are issued before the
 // MFMAs of step k.
-#include "common.hpp"
-#include "internal.hpp"
+#include "gemm_core.hpp"
 
 namespace lssm {
 
 namespace {
 
 constexpr int BM = 128, BN = 128, BK = 64, PAD = 72, NT = 256;
-
-template <typename T> struct MfmaOp;
-template <> struct MfmaOp<f16> {
-    using frag = half8;
-    static __device__ __forceinline__ floatx16 mma(frag a, frag b, floatx16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-};
-template <> struct MfmaOp<bf16> {
-    using frag = bf16x8;
-    static __device__ __forceinline__ floatx16 mma(frag a, frag b, floatx16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-};
 
 // Per-thread register staging of one K step.
 template <int FMT> struct BStage {
@@ -237,117 +222,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(GemmArgs a) {
 // elements (128 B) whose 16-byte slots are XOR-swizzled by swz(row), so the
 // fragment reads of 16 consecutive rows hit distinct banks without padding.
 // ---------------------------------------------------------------------------
-constexpr int G2M = 256, G2K = 64;
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// 16 consecutive quantized weights of one row: raw bits + fp16 scale bits.
-template <int FMT> struct WRaw { u32x2 q; uint32_t s; };
-template <> struct WRaw<LSSM_W_Q8_G32> { u32x4 q; uint32_t s; };
-
-template <typename T> __device__ __forceinline__ uint32_t pk2(float lo, float hi) {
-    if constexpr (__is_same(T, bf16)) {
-        typedef __bf16 v2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, v2{(__bf16)lo, (__bf16)hi});
-    } else {
-        typedef _Float16 v2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, v2{from_f<f16>(lo), from_f<f16>(hi)});
-    }
-}
-
-// r(q s) for 8 consecutive weights -> 4 packed pairs (k order).  The
-// unsigned value u (int4: q + 8, int8: q + 128) of two weights is placed by
-// one v_perm into the mantissas of two fp16 values 1024 + u (bits
-// 0x6400 | u), and fma(1024 + u, s, c) with c = -(1024 + 8) s (int8:
-// -(1024 + 128) s) is q s exactly: both products have at most 11 + 11
-// significant bits and q s at most 15, all exact in fp32; the fp16 operands
-// convert inside v_fma_mix_f32.  One rounding, at the pack.  int4: q0 holds
-// the 8 nibbles (k = nibble index); int8: q0, q1 the 8 bytes.
-template <int FMT, typename T>
-__device__ __forceinline__ u32x4 dequant8(uint32_t q0, uint32_t q1, float s, float c) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    // bytes (b0 of v, 0x64, b1 of v, 0x64) and (b2, 0x64, b3, 0x64)
-    auto pair01 = [](uint32_t v) { return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)); };
-    auto pair23 = [](uint32_t v) { return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)); };
-    auto f = [&](_Float16 e) { return __builtin_fmaf((float)e, s, c); };
-    if constexpr (FMT == LSSM_W_Q8_G32) {
-        const uint32_t d0 = q0 ^ 0x80808080u, d1 = q1 ^ 0x80808080u;
-        const h2 a = pair01(d0), b = pair23(d0), e = pair01(d1), g = pair23(d1);
-        return u32x4{pk2<T>(f(a.x), f(a.y)), pk2<T>(f(b.x), f(b.y)), pk2<T>(f(e.x), f(e.y)), pk2<T>(f(g.x), f(g.y))};
-    } else {
-        // u of k 0, 2, 4, 6 (low nibbles) and k 1, 3, 5, 7
-        const uint32_t lo = (q0 & 0x0F0F0F0Fu) ^ 0x08080808u;
-        const uint32_t hi = ((q0 >> 4) & 0x0F0F0F0Fu) ^ 0x08080808u;
-        const h2 e02 = pair01(lo), e46 = pair23(lo), e13 = pair01(hi), e57 = pair23(hi);
-        return u32x4{pk2<T>(f(e02.x), f(e13.x)), pk2<T>(f(e02.y), f(e13.y)),
-                     pk2<T>(f(e46.x), f(e57.x)), pk2<T>(f(e46.y), f(e57.y))};
-    }
-}
-template <int FMT> __device__ __forceinline__ float dequant_bias(float s) {
-    return (FMT == LSSM_W_Q8_G32 ? -1152.0f : -1032.0f) * s;
-}
-
-// 16 weights -> 8 packed pairs
-template <int FMT, typename T>
-__device__ __forceinline__ void dequant16(const WRaw<FMT>& r, uint32_t out[8]) {
-    const float s = fp16_bits_to_f((uint16_t)r.s), c = dequant_bias<FMT>(s);
-    u32x4 a, b;
-    if constexpr (FMT == LSSM_W_Q8_G32) {
-        a = dequant8<FMT, T>(r.q[0], r.q[1], s, c);
-        b = dequant8<FMT, T>(r.q[2], r.q[3], s, c);
-    } else {
-        a = dequant8<FMT, T>(r.q[0], 0u, s, c);
-        b = dequant8<FMT, T>(r.q[1], 0u, s, c);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        out[i] = a[i];
-        out[4 + i] = b[i];
-    }
-}
-
-__device__ __forceinline__ void lds_dma16(const void* g, void* l) {
-    __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)l, 16, 0, 0);
-}
-// The same DMA as inline asm, for waves that also read LDS: the compiler does
-// not see it, so it does not wait for it before every LDS read (it cannot
-// tell which LDS bytes a DMA writes); the issuing wave waits with an explicit
-// vmcnt.  m0 (the LDS base of the 1 KiB run) is saved and restored.
-__device__ __forceinline__ void lds_dma16_asm(const void* g, uint32_t lds_byte) {
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(g), "s"(lds_byte)
-        : "memory");
-}
-template <typename T> __device__ __forceinline__ uint32_t lds_addr(const T* p) {
-    return (uint32_t)(size_t)((const __attribute__((address_space(3))) T*)p);
-}
-
-// LDS tile rows are 128 B (64 16-bit elements, 8 slots of 16 B) and the
-// banks repeat every 256 B, so rows r and r + 2 share banks.  Physical slot =
-// logical slot ^ ((r / 2) % 8): 16 consecutive rows read or written at one
-// logical slot then cover all 16 16-byte positions of the 256 B window (row
-// parity picks the half, the XOR the position), with no bank conflict.
-__device__ __forceinline__ constexpr uint32_t swz(uint32_t row) { return (row >> 1) & 7u; }
-
-// Workgroups go to the 8 XCDs round-robin in launch order (linear id % 8),
-// and each XCD has its own L2.  Give XCD x a contiguous run of the tiles in
-// M-major order, so the blocks that share an X row block (all N tiles of one
-// M tile) run on one XCD and read X through one L2.  A bijection for any grid.
-__device__ __forceinline__ void xcd_tile(uint32_t& mt, uint32_t& nt) {
-    const uint32_t nbx = gridDim.x, total = nbx * gridDim.y;
-    const uint32_t lin = blockIdx.x + nbx * blockIdx.y;
-    const uint32_t x = lin % 8, q = total / 8, r = total % 8;
-    const uint32_t tile = x * q + min(x, r) + lin / 8;
-    mt = tile / nbx;
-    nt = tile % nbx;
-}
+constexpr int G2M = 256;
 
 // CW compute waves: 4 -> 256 x 128 tile, 8 -> 256 x 256 (quantized W only:
 // the LDS is then exactly full, 3 x 32 KiB of X + 2 x 32 KiB of W).
@@ -370,9 +245,7 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
     uint32_t tm, tn;
     xcd_tile(tm, tn);
     const uint32_t m0 = tm * G2M, n0 = tn * BN;
-    // split K (gridDim.z > 1, small grids): slice z takes steps z KT .. + KT
-    // and writes its fp32 sums to a.ws; K stays the row length of X and W
-    const uint32_t K = a.K, KT = K / G2K / gridDim.z, kz = blockIdx.z * KT * G2K;
+    const uint32_t K = a.K, KT = K / G2K;
     // a barrier without __syncthreads' release fence (which would wait for
     // every DMA in flight); the empty asm keeps memory operations in place
     auto barrier = [] {
@@ -394,7 +267,7 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
             for (int j = 0; j < 4; ++j) {
                 const uint32_t sl = (lane % 8) ^ swz(8 * j + lane / 8);
                 const uint32_t n = min(n0 + 32 * q + 8 * j + lane / 8, a.N - 1);
-                wq[j] = (const char*)a.w + ((size_t)n * K + kz + 8 * sl) * sizeof(T);
+                wq[j] = (const char*)a.w + ((size_t)n * K + 8 * sl) * sizeof(T);
             }
             auto dma_w = [&](uint32_t kt) {
                 T* dst = Bs[kt % SB] + (32 * q) * G2K;
@@ -422,9 +295,8 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
             const uint32_t br = p / TPR, c0 = (p % TPR) * CPT;
             constexpr uint32_t GS = FMT == LSSM_W_Q4_G64 ? 64 : 32;
             const uint32_t nrow = min(n0 + br, a.N - 1);
-            const char* wq = (const char*)a.w + (size_t)nrow * (FMT == LSSM_W_Q8_G32 ? K : K / 2) +
-                             (FMT == LSSM_W_Q8_G32 ? kz : kz / 2);
-            const uint16_t* sp = (const uint16_t*)a.s + (size_t)nrow * (K / GS) + kz / GS;
+            const char* wq = (const char*)a.w + (size_t)nrow * (FMT == LSSM_W_Q8_G32 ? K : K / 2);
+            const uint16_t* sp = (const uint16_t*)a.s + (size_t)nrow * (K / GS);
             using R = WRaw<FMT>;
             auto load_w = [&](uint32_t kt, R (&r)[CPT]) {
 #pragma unroll
@@ -489,7 +361,7 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
     }
     const uint32_t as0 = lds_addr(&As[0][0]) + (XR * w) * G2K * (uint32_t)sizeof(T);
     auto dma_x = [&](uint32_t kt, int j0, int j1) {
-        const char* base = (const char*)a.x + ((size_t)kz + (size_t)kt * G2K) * sizeof(T);
+        const char* base = (const char*)a.x + (size_t)kt * G2K * sizeof(T);
         const uint32_t dst = as0 + (kt % 3) * (G2M * G2K * (uint32_t)sizeof(T));
         for (int j = j0; j < j1; ++j) lds_dma16_asm(base + xo[j], dst + 8 * j * G2K * (uint32_t)sizeof(T));
     };
@@ -499,7 +371,7 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
     // each row's from its lane by readlane instead of waiting, per 32-row
     // block, on 16 scattered loads
     float rs_lo = 1.0f, rs_hi = 1.0f;
-    if (a.row_scale && gridDim.z == 1) {
+    if (a.row_scale) {
         const uint32_t mb = m0 + wm * 128;
         rs_lo = a.row_scale[min(mb + lane, a.M - 1)];
         rs_hi = a.row_scale[min(mb + 64 + lane, a.M - 1)];
@@ -571,22 +443,6 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
 
     // D layout of v_mfma_f32_32x32x*: element r of lane l is
     // row (r/4)*8 + (l/32)*4 + r%4, column l%32.
-    if (gridDim.z > 1) {
-        float* ws = a.ws + (size_t)blockIdx.z * a.M * a.N;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t n = n0 + wn * 64 + j * 32 + lane % 32;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t m = m0 + wm * 128 + i * 32 + (r / 4) * 8 + (lane / 32) * 4 + r % 4;
-                    if (m < a.M && n < a.N) ws[(size_t)m * a.N + n] = acc[i][j][r];
-                }
-            }
-        }
-        return;
-    }
     T* Y = (T*)a.y;
     const T* Rz = (const T*)a.res;
     const bool vec = a.y_stride % 8 == 0 && (uintptr_t)a.y % 16 == 0 &&
@@ -922,95 +778,56 @@ hipError_t go_skinny_mt(hipStream_t s, const GemmArgs& a, int upw) {
     return go_skinny<FMT, T, MT, 1>(s, a);
 }
 
-// The split slices' fp32 sums added in slice order, then gemm2_kernel's
-// epilogue: r(v), r(silu(v)) or r(res + r(v)).
-template <typename T, int EPI>
-__global__ __launch_bounds__(256) void gemm_split_sum_kernel(GemmArgs a, uint32_t S) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, MN = (size_t)a.M * a.N;
-    if (i >= MN) return;
-    float v = 0.0f;
-    for (uint32_t z = 0; z < S; ++z) v += a.ws[z * MN + i];
-    const uint32_t m = (uint32_t)(i / a.N), n = (uint32_t)(i % a.N);
-    const size_t yi = (size_t)m * a.y_stride + n;
-    if (a.row_scale) v *= a.row_scale[m];
-    if (n < a.silu_cols) v = silu_fast(v);
-    if (EPI == LSSM_EPI_SILU) v = silu_f(v);
-    if (EPI == LSSM_EPI_ADD) v = to_f(((const T*)a.res)[yi]) + rnd<T>(v);
-    ((T*)a.y)[yi] = from_f<T>(v);
+// gemm2_kernel's tiles for a call.  256-wide tiles halve the X re-reads: a wide
+// tile takes about 1.5x the time of a 128-wide one (measured at the 2.7B
+// out_proj shape), so they are taken when their rounds of blocks (one block per
+// CU) cost less: 1.5 ceil(wide tiles / CUs) <= ceil(narrow tiles / CUs)
+struct Gemm2Rounds {
+    bool wide;
+    uint64_t cost;   // estimate as gemm_mid_plan's: 8 us a round and 0.78 a K step of narrow tiles, 1.5 of wide ones
+};
+inline Gemm2Rounds gemm2_rounds(const GemmArgs& a) {
+    const uint64_t cus = num_cus(), mt = (a.M + G2M - 1) / G2M;
+    const uint64_t rw = (mt * ((a.N + 255) / 256) + cus - 1) / cus, rn = (mt * ((a.N + 127) / 128) + cus - 1) / cus;
+    const bool wide = a.wfmt != LSSM_W_DENSE && 3 * rw <= 2 * rn;
+    return {wide, 200 + (wide ? rw : rn) * (800 + (a.K / G2K) * (wide ? 150 : 78))};
 }
 
-// The same, four consecutive outputs a thread (N and the row strides
-// multiples of 4): 16-byte loads of the slices' sums.
-template <typename T, int EPI>
-__global__ __launch_bounds__(256) void gemm_split_sum4_kernel(GemmArgs a, uint32_t S) {
-    const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x, MN = (size_t)a.M * a.N;
-    if (4 * q >= MN) return;
-    floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t z = 0; z < S; ++z) {
-        const floatx4 p = reinterpret_cast<const floatx4*>(a.ws + z * MN)[q];
-        v[0] += p[0];
-        v[1] += p[1];
-        v[2] += p[2];
-        v[3] += p[3];
-    }
-    const uint32_t m = (uint32_t)(4 * q / a.N), n = (uint32_t)(4 * q % a.N);
-    const size_t yi = (size_t)m * a.y_stride + n;
-    T o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        float x = v[e];
-        if (a.row_scale) x *= a.row_scale[m];
-        if (n + e < a.silu_cols) x = silu_fast(x);
-        if (EPI == LSSM_EPI_SILU) x = silu_f(x);
-        if (EPI == LSSM_EPI_ADD) x = to_f(((const T*)a.res)[yi + e]) + rnd<T>(x);
-        o[e] = from_f<T>(x);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ((T*)a.y)[yi + e] = o[e];
+// Whether a call goes to gemm_mid's smaller tiles: up to 128 rows, except dense
+// grids well past the CUs (the lm_head), where gemm_kernel's 128 x 128 tiles
+// stream W as fast (50280 x 2560 at 16 rows: 57 us against 60); above, where
+// their estimate is below gemm2_kernel's.
+inline bool gemm_takes_mid(const GemmArgs& a) {
+    const GemmMidPlan p = gemm_mid_plan(a);
+    if (!p.bm) return false;
+    if (a.M <= 128) return a.wfmt != LSSM_W_DENSE || 2 * (uint64_t)((a.N + 127) / 128) < 3 * (uint64_t)num_cus();
+    return p.cost < gemm2_rounds(a).cost;
 }
 
-// K slices for a prefill GEMM whose 256 x 128 tiles would leave most CUs idle
-// (the 130M out_proj at 2048 rows: 48 tiles): as many as fill about half the
-// CUs, K / 64 divisible, the workspace large enough; 1 = no split.
-inline uint32_t gemm_split(const GemmArgs& a, uint32_t gs) {
-    static const bool off = [] {
-        const char* v = getenv("LSSM_GEMM_SPLIT");
-        return v && v[0] == '0';
-    }();
-    if (!a.ws || off) return 1;
-    const size_t narrow = (size_t)((a.M + G2M - 1) / G2M) * ((a.N + 127) / 128), cus = num_cus();
-    if (2 * narrow > cus) return 1;
-    uint32_t S = 1;
-    for (uint32_t c : {2u, 4u, 8u})
-        if (narrow * c <= cus && (a.K / G2K) % c == 0 && (a.K / c) % gs == 0 &&
-            (size_t)c * a.M * a.N <= a.ws_floats)
-            S = c;
-    return S;
+// Units per wave of the skinny kernel for a call, 0 where it does not take it:
+// few rows, weights streamed once.  Every block reads all of x, so past 16 rows
+// only while that is small: 37 x 10576 x 2560 int4 26.2 us against 15.2 in
+// gemm_mid, 32 x 768 x 1536 int8 8.4 against 9.2, 37 x 3352 x 768 int8 6.6
+// against 7.5 (64 rows: 7.8 against 7.6).
+template <int FMT> int skinny_takes(const GemmArgs& a) {
+    if (a.M > 48 || (a.M > 32 && a.K > 1024) || (a.M > 16 && a.K > 2048)) return 0;
+    return skinny_upw<FMT>(a.K, (int)(a.M + 15) / 16);
 }
 
 template <int FMT, typename T>
 hipError_t go_epi(hipStream_t s, const GemmArgs& a) {
-    // decode batches: weights streamed once
-    if (a.M <= 64) {
-        const int mt = a.M <= 16 ? 1 : (a.M <= 32 ? 2 : 4);
-        if (const int upw = skinny_upw<FMT>(a.K, mt)) {
-            if (mt == 1) return go_skinny_mt<FMT, T, 1>(s, a, upw);
-            if (mt == 2) return go_skinny_mt<FMT, T, 2>(s, a, upw);
-            return go_skinny_mt<FMT, T, 4>(s, a, upw);
-        }
+    if (const int upw = skinny_takes<FMT>(a)) {
+        if (a.M <= 16) return go_skinny_mt<FMT, T, 1>(s, a, upw);
+        if (a.M <= 32) return go_skinny_mt<FMT, T, 2>(s, a, upw);
+        return go_skinny_mt<FMT, T, 3>(s, a, upw);
     }
+    if (gemm_takes_mid(a)) return launch_gemm_mid(s, a, gemm_mid_plan(a));
     // the large tile for prefill-sized M; X byte offsets within a 256-row
     // tile fit 32 bits
     if (a.M > 128 && (uint64_t)a.M * a.x_stride * sizeof(T) < (1ull << 31)) {
-        // 256-wide tiles halve the X re-reads: a wide tile takes about 1.5x
-        // the time of a 128-wide one (measured at the 2.7B out_proj shape),
-        // so take them when their rounds of blocks (one block per CU) cost
-        // less: 1.5 ceil(wide tiles / CUs) <= ceil(narrow tiles / CUs)
         const uint32_t mt = (a.M + G2M - 1) / G2M;
         const size_t cus = num_cus();
-        const size_t rw = (mt * (size_t)((a.N + 255) / 256) + cus - 1) / cus;
-        const size_t rn = (mt * (size_t)((a.N + 127) / 128) + cus - 1) / cus;
-        const bool wide = FMT != LSSM_W_DENSE && 3 * rw <= 2 * rn;
+        const bool wide = gemm2_rounds(a).wide;
         auto run_wide = [&](const GemmArgs& g) {
             dim3 grid((g.N + 255) / 256, mt);
             if constexpr (FMT != LSSM_W_DENSE) {
@@ -1021,30 +838,6 @@ hipError_t go_epi(hipStream_t s, const GemmArgs& a) {
                 }
             }
         };
-        const uint32_t S = FMT == LSSM_W_DENSE ? 1u : gemm_split(a, FMT == LSSM_W_Q4_G64 ? 64u : 32u);
-        if (S > 1) {
-            // small grid: K in S slices, then the slices' sums (one launch)
-            dim3 grid((a.N + 127) / 128, mt, S);
-            gemm2_kernel<FMT, T, LSSM_EPI_NONE, 4><<<grid, 512, 0, s>>>(a);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-            if (a.N % 4 == 0 && (uintptr_t)a.ws % 16 == 0) {
-                const unsigned nb = (unsigned)(((size_t)a.M * a.N / 4 + 255) / 256);
-                switch (a.epi) {
-                    case LSSM_EPI_SILU: gemm_split_sum4_kernel<T, LSSM_EPI_SILU><<<nb, 256, 0, s>>>(a, S); break;
-                    case LSSM_EPI_ADD: gemm_split_sum4_kernel<T, LSSM_EPI_ADD><<<nb, 256, 0, s>>>(a, S); break;
-                    default: gemm_split_sum4_kernel<T, LSSM_EPI_NONE><<<nb, 256, 0, s>>>(a, S); break;
-                }
-                return hipGetLastError();
-            }
-            const unsigned nb = (unsigned)(((size_t)a.M * a.N + 255) / 256);
-            switch (a.epi) {
-                case LSSM_EPI_SILU: gemm_split_sum_kernel<T, LSSM_EPI_SILU><<<nb, 256, 0, s>>>(a, S); break;
-                case LSSM_EPI_ADD: gemm_split_sum_kernel<T, LSSM_EPI_ADD><<<nb, 256, 0, s>>>(a, S); break;
-                default: gemm_split_sum_kernel<T, LSSM_EPI_NONE><<<nb, 256, 0, s>>>(a, S); break;
-            }
-            return hipGetLastError();
-        }
         auto run_narrow = [&](const GemmArgs& g) {
             dim3 grid((g.N + 127) / 128, mt);
             switch (g.epi) {
@@ -1122,8 +915,24 @@ bool gemm_norm_fold_takes(const GemmArgs& a) {
     if (a.N % 128 != 0 || a.y_stride % 8 != 0) return false;
     for (const void* p : {(const void*)a.y, a.res, (const void*)a.y2, a.y2_w})
         if ((uintptr_t)p % 16 != 0) return false;
-    if (a.wfmt != LSSM_W_DENSE && gemm_split(a, a.wfmt == LSSM_W_Q4_G64 ? 64u : 32u) > 1) return false;
-    return true;
+    GemmArgs b = a;                              // a call that takes gemm_mid's tiles is not folded
+    b.y2 = nullptr;
+    return !gemm_takes_mid(b);
+}
+
+bool gemm_wants_ws(const GemmArgs& a) {
+    int skinny;
+    switch (a.wfmt) {
+        case LSSM_W_Q4_B32: skinny = skinny_takes<LSSM_W_Q4_B32>(a); break;
+        case LSSM_W_Q4_G64: skinny = skinny_takes<LSSM_W_Q4_G64>(a); break;
+        case LSSM_W_Q8_G32: skinny = skinny_takes<LSSM_W_Q8_G32>(a); break;
+        default: skinny = skinny_takes<LSSM_W_DENSE>(a); break;
+    }
+    if (a.act == LSSM_F32 || skinny) return false;
+    GemmArgs b = a;
+    b.ws = reinterpret_cast<float*>(16);
+    b.ws_floats = GEMM_WS_FLOATS;
+    return gemm_takes_mid(b) && gemm_mid_plan(b).split > 1;
 }
 
 hipError_t launch_gemm(hipStream_t s, const GemmArgs& a) {

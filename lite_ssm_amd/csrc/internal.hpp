@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -36,8 +37,14 @@ struct lssm_ctx {
     float* ssd_gram = nullptr;
     size_t ssd_gram_cap = 0;   // floats
     std::vector<float*> ssd_gram_retired;
+    // split-K slices of lssm_linear's GEMM (lssm::GEMM_WS_FLOATS), allocated by
+    // the first call that splits outside a stream capture
+    float* gemm_ws = nullptr;
     // x rows packed for the batched decode GEMV (lssm::GEMV_PACK_BYTES)
     void* xpack = nullptr;
+    // held while a call enqueues the launches that pass gemm_ws or xpack on to
+    // each other (two threads on one context)
+    std::mutex scratch_mu;
 };
 
 namespace lssm {
@@ -215,12 +222,22 @@ struct GemmArgs {
 // N % 128 == 0, 16-byte aligned rows.  launch_gemm refuses y2 elsewhere.
 bool gemm_norm_fold_takes(const GemmArgs& a);
 hipError_t launch_gemm(hipStream_t s, const GemmArgs& a);
-// Workspace the engine gives launch_gemm for its split-K slices (floats).
-// The 130M prefill of 2048 tokens (config 3) runs its out_proj in four slices
-// plus the sum: 2.60 -> 2.45 ms for the whole prefill; the same GEMM alone
-// through lssm_linear (no workspace) measures 23.9 us unsplit against 26.5 us
-// split, so the generic entry keeps the single launch.
+// Workspace the engine and the contexts give launch_gemm for its split-K
+// slices (floats).
 constexpr size_t GEMM_WS_FLOATS = (size_t)8 << 20;   // 32 MiB
+// The same product in smaller tiles (gemm_mid.hip) for grids that leave CUs
+// idle: bm x bn tiles, K in `split` slices (more than one only with a.ws) and
+// an estimate of its time; cost ~0 and bm 0 where it does not take the call.
+struct GemmMidPlan {
+    int bm = 0, bn = 0;
+    uint32_t split = 1;
+    uint64_t cost = ~0ull;
+};
+GemmMidPlan gemm_mid_plan(const GemmArgs& a);
+hipError_t launch_gemm_mid(hipStream_t s, const GemmArgs& a, const GemmMidPlan& p);
+// Whether launch_gemm would split K if a.ws were a workspace of
+// GEMM_WS_FLOATS.
+bool gemm_wants_ws(const GemmArgs& a);
 // GEMM for fp32 activations (any row count) and for operands the MFMA GEMMs'
 // 16-byte loads cannot take: fp32 on the fp32 MFMA where gemm_f32_takes says
 // so, else one thread per output.

@@ -126,3 +126,46 @@ def test_gemv_int8_bf16(ctx, rng, M, K):
     ctx.linear(dev(x), dev(w), dev(s), y, M, N, K, O.W_Q8_G32, act)
     ref = O.linear(x, w, s, M, N, K, O.W_Q8_G32, act)
     assert_close(act_host(y, act), ref, act, 1.6e-2, "gemv")
+
+
+# --------------------------------------------------------------------------- small-tile GEMM
+# Rows at the edges of the 64- and 128-row tiles, partial tiles in N, depths of
+# 1, 2, 3, 5 and 13 K steps, K deep enough to be split, and enough columns for
+# each of the three tiles; the largest has more tiles than CUs.
+@pytest.mark.parametrize("act", [O.F16, O.BF16])
+@pytest.mark.parametrize("wfmt", ALL_FMTS)
+@pytest.mark.parametrize("M,N,K", [(33, 200, 64), (63, 72, 1088), (64, 64, 128), (65, 130, 192), (127, 500, 320),
+                                   (129, 1000, 832), (300, 1100, 2560), (17, 40, 5120), (12, 300, 8192),
+                                   (100, 9000, 192), (300, 6000, 128), (700, 2560, 320), (1000, 2000, 128)])
+def test_small_tile_gemm_vs_oracle(ctx, rng, act, wfmt, M, N, K):
+    print(f"case: small-tile GEMM act {act} fmt {wfmt} {M} x {N} x {K}", flush=True)
+    x = O.to_act(rng.standard_normal((M, K)), act)
+    w, s = _weights(rng, N, K, wfmt, act)
+    y = empty((M, N), act)
+    ctx.linear(dev(x), dev(w), _sdev(s), y, M, N, K, wfmt, act)
+    ref = O.linear(x, w, s, M, N, K, wfmt, act, round_dequant=1)
+    assert_close(act_host(y, act), ref, act, {O.F16: 2e-3, O.BF16: 1.6e-2}[act], "small-tile gemm")
+
+
+@pytest.mark.parametrize("act", [O.F16, O.BF16])
+@pytest.mark.parametrize("M,N,K", [(37, 130, 192), (70, 256, 5120)])
+def test_small_tile_gemm_strides_epilogues(ctx, rng, act, M, N, K):
+    """Padded rows (an odd y stride: element stores), SiLU and the in-place
+    residual, in one pass and (K = 5120) through the slices' sum."""
+    import lite_ssm_amd as L
+    for wfmt in (O.W_DENSE, O.W_Q4_G64):
+        w, s = _weights(rng, N, K, wfmt, act)
+        xp = O.to_act(rng.standard_normal((M, K + 8)), act)
+        x = np.ascontiguousarray(xp[:, :K])
+        for pad in (8, 3):
+            res = O.to_act(rng.standard_normal((M, N + pad)), act)
+            for epi in (L.EPI_NONE, L.EPI_SILU, L.EPI_ADD):
+                print(f"case: small-tile GEMM strided act {act} fmt {wfmt} {M} x {N} x {K} pad {pad} epi {epi}", flush=True)
+                y = dev(res)
+                ctx.linear(dev(xp), dev(w), _sdev(s), y, M, N, K, wfmt, act, epi=epi,
+                           residual=y if epi == L.EPI_ADD else None, x_stride=K + 8, y_stride=N + pad)
+                ref = O.linear(x, w, s, M, N, K, wfmt, act, epi=epi, round_dequant=1,
+                               residual=np.ascontiguousarray(res[:, :N]) if epi == L.EPI_ADD else None)
+                got = act_host(y, act)
+                assert_close(np.ascontiguousarray(got[:, :N]), ref, act, {O.F16: 2e-3, O.BF16: 1.6e-2}[act], "epilogue")
+                assert np.array_equal(got[:, N:], res[:, N:])
