@@ -782,15 +782,26 @@ hipError_t go_skinny_mt(hipStream_t s, const GemmArgs& a, int upw) {
 // tile takes about 1.5x the time of a 128-wide one (measured at the 2.7B
 // out_proj shape), so they are taken when their rounds of blocks (one block per
 // CU) cost less: 1.5 ceil(wide tiles / CUs) <= ceil(narrow tiles / CUs)
-struct Gemm2Rounds {
+//
+// A last round of wide tiles at most half full (2.7B out_proj: 640 tiles = 2.5
+// rounds) runs instead as one round of narrow tiles: the columns of the full
+// rounds (wide_n) go to the wide launch, the rest to a narrow one.
+struct Gemm2Plan {
     bool wide;
-    uint64_t cost;   // estimate as gemm_mid_plan's: 8 us a round and 0.78 a K step of narrow tiles, 1.5 of wide ones
+    uint32_t wide_n;   // columns of the wide launch (N: all)
+    uint64_t cost;     // as gemm_mid_plan's: a round 8 us and per K step 0.78 (narrow) or 1.6 (wide)
 };
-inline Gemm2Rounds gemm2_rounds(const GemmArgs& a) {
-    const uint64_t cus = num_cus(), mt = (a.M + G2M - 1) / G2M;
-    const uint64_t rw = (mt * ((a.N + 255) / 256) + cus - 1) / cus, rn = (mt * ((a.N + 127) / 128) + cus - 1) / cus;
-    const bool wide = a.wfmt != LSSM_W_DENSE && 3 * rw <= 2 * rn;
-    return {wide, 200 + (wide ? rw : rn) * (800 + (a.K / G2K) * (wide ? 150 : 78))};
+inline Gemm2Plan gemm2_plan(const GemmArgs& a) {
+    const uint64_t cus = num_cus(), mt = (a.M + G2M - 1) / G2M, KT = a.K / G2K;
+    const uint64_t wt = mt * ((a.N + 255) / 256), nt = mt * ((a.N + 127) / 128);
+    const uint64_t rw = (wt + cus - 1) / cus, rn = (nt + cus - 1) / cus;
+    if (a.wfmt == LSSM_W_DENSE || 3 * rw > 2 * rn) return {false, 0, 200 + rn * (800 + 78 * KT)};
+    const uint64_t full = wt / cus, rem = wt % cus;
+    const uint32_t n1 = (uint32_t)(full * cus / mt) * 256u;
+    const bool split = full >= 1 && rem > 0 && 2 * rem <= cus && n1 > 0 && n1 < a.N &&
+                       mt * ((a.N - n1 + 127) / 128) <= cus;
+    if (!split) return {true, a.N, 200 + rw * (800 + 160 * KT)};
+    return {true, n1, 400 + full * (800 + 160 * KT) + 800 + 78 * KT};
 }
 
 // Whether a call goes to gemm_mid's smaller tiles: up to 128 rows, except dense
@@ -801,7 +812,7 @@ inline bool gemm_takes_mid(const GemmArgs& a) {
     const GemmMidPlan p = gemm_mid_plan(a);
     if (!p.bm) return false;
     if (a.M <= 128) return a.wfmt != LSSM_W_DENSE || 2 * (uint64_t)((a.N + 127) / 128) < 3 * (uint64_t)num_cus();
-    return p.cost < gemm2_rounds(a).cost;
+    return p.cost < gemm2_plan(a).cost;
 }
 
 // Units per wave of the skinny kernel for a call, 0 where it does not take it:
@@ -826,8 +837,7 @@ hipError_t go_epi(hipStream_t s, const GemmArgs& a) {
     // tile fit 32 bits
     if (a.M > 128 && (uint64_t)a.M * a.x_stride * sizeof(T) < (1ull << 31)) {
         const uint32_t mt = (a.M + G2M - 1) / G2M;
-        const size_t cus = num_cus();
-        const bool wide = gemm2_rounds(a).wide;
+        const Gemm2Plan plan = gemm2_plan(a);
         auto run_wide = [&](const GemmArgs& g) {
             dim3 grid((g.N + 255) / 256, mt);
             if constexpr (FMT != LSSM_W_DENSE) {
@@ -846,22 +856,14 @@ hipError_t go_epi(hipStream_t s, const GemmArgs& a) {
                 default: gemm2_kernel<FMT, T, LSSM_EPI_NONE, 4><<<grid, 512, 0, s>>>(g); break;
             }
         };
-        if (wide) {
-            // A last round of wide tiles at most half full (2.7B out_proj: 640
-            // tiles = 2.5 rounds) runs instead as one round of narrow tiles,
-            // which take about two thirds of a wide tile's time: the columns of
-            // the full rounds go to the wide launch, the rest to a narrow one
-            // (pointers offset by whole output columns, so each output is
-            // computed exactly as in the single launch).
-            const size_t wt = mt * (size_t)((a.N + 255) / 256);
-            const size_t full = wt / cus, rem = wt % cus;
-            const uint32_t n1 = full ? (uint32_t)((full * cus) / mt) * 256u : 0u;
-            const bool split = full >= 1 && rem > 0 && 2 * rem <= cus && n1 > 0 && n1 < a.N &&
-                               mt * (size_t)((a.N - n1 + 127) / 128) <= cus;
-            if (!split) {
+        if (plan.wide) {
+            const uint32_t n1 = plan.wide_n;
+            if (n1 >= a.N) {
                 run_wide(a);
                 return hipGetLastError();
             }
+            // (pointers offset by whole output columns, so each output is
+            // computed exactly as in a single launch)
             GemmArgs a1 = a, a2 = a;
             a1.N = n1;
             a2.N = a.N - n1;
