@@ -8,6 +8,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "conv_core.hpp"
 #include "internal.hpp"
 
 namespace lssm {
@@ -25,22 +26,6 @@ namespace lssm {
             __VA_ARGS__;                                 \
         }                                                \
     } while (0)
-
-// 8 fp16 / bf16 values in a 16-byte vector register.
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-template <typename T> __device__ __forceinline__ float el8(v4u v, int e) {
-    const uint32_t d = v[e / 2];
-    return f_of_bits<T>((uint16_t)((e & 1) ? (d >> 16) : (d & 0xFFFF)));
-}
-template <typename T> __device__ __forceinline__ uint32_t bits_t(float f) {
-    return __builtin_bit_cast(uint16_t, from_f<T>(f));
-}
-template <typename T> __device__ __forceinline__ v4u pack8(const float (&f)[8]) {
-    v4u r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = bits_t<T>(f[2 * i]) | (bits_t<T>(f[2 * i + 1]) << 16);
-    return r;
-}
 
 constexpr int NT = 256;
 
@@ -249,59 +234,12 @@ __global__ __launch_bounds__(256) void conv1d_vec_kernel(const T* __restrict__ x
     if (d0 >= D) return;
     const uint32_t t0 = blockIdx.y * CONV_CT;
     const uint32_t b = blockIdx.z;
-    const T* xb = x + (size_t)b * L * xs + d0;
-    // the window as vector registers; elements are taken out by shifts (an
-    // element address would put the array in scratch memory)
     v4u win[CONV_CT + 3];
-#pragma unroll
-    for (int i = 0; i < CONV_CT + 3; ++i) {
-        const int t = (int)t0 + i - 3;
-        win[i] = (t >= 0 && t < (int)L) ? *reinterpret_cast<const v4u*>(xb + (size_t)t * xs)
-                                        : v4u{0, 0, 0, 0};
-    }
-    // rows before the first (t0 == 0 only): the sequence's earlier rows, the
-    // last K entries of each channel's conv state (entry K + t for row t < 0)
-    if (hist && t0 == 0) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            uint32_t h[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint16_t lo = __builtin_bit_cast(uint16_t, hist[(size_t)(d0 + 2 * q) * 4 + 1 + i]);
-                const uint16_t hi = __builtin_bit_cast(uint16_t, hist[(size_t)(d0 + 2 * q + 1) * 4 + 1 + i]);
-                h[q] = (uint32_t)lo | ((uint32_t)hi << 16);
-            }
-            win[i] = v4u{h[0], h[1], h[2], h[3]};
-        }
-    }
-    // taps w[d][0..3] of the 8 channels: 64 contiguous bytes
-    float wf[8][4], bf[8];
-    {
-        const v4u* w4 = reinterpret_cast<const v4u*>(w + (size_t)d0 * 4);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const v4u v = w4[q];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) wf[2 * q + e / 4][e % 4] = el8<T>(v, e);
-        }
-        const v4u bv = bias ? *reinterpret_cast<const v4u*>(bias + d0) : v4u{0, 0, 0, 0};
-#pragma unroll
-        for (int c = 0; c < 8; ++c) bf[c] = el8<T>(bv, c);
-    }
+    conv_window<T, CONV_CT>(x + (size_t)b * L * xs + d0, xs, t0, L, hist ? hist + (size_t)d0 * 4 : nullptr, win);
     T* yb = y + ((size_t)b * L + t0) * ys + d0;
-#pragma unroll
-    for (int i = 0; i < CONV_CT; ++i) {
-        float o[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            float acc = bf[c];
-#pragma unroll
-            for (int tap = 0; tap < 4; ++tap) acc = fmaf(wf[c][tap], el8<T>(win[i + tap], c), acc);
-            o[c] = rnd<T>(acc);
-            if (SILU) o[c] = silu_fast(o[c]);
-        }
-        if (t0 + i < L) *reinterpret_cast<v4u*>(yb + (size_t)i * ys) = pack8<T>(o);
-    }
+    conv_rows<T, CONV_CT, SILU>(win, w + (size_t)d0 * 4, bias ? bias + d0 : nullptr, [&](int i, v4u o) {
+        if (t0 + i < L) *reinterpret_cast<v4u*>(yb + (size_t)i * ys) = o;
+    });
   }
 }
 

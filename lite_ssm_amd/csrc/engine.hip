@@ -557,11 +557,15 @@ struct lssm_engine {
             } else {
                 const char* xbc_pre = prj + (size_t)d_inner * es;
                 if (wait) e = hipStreamWaitEvent(strm, wait[li], 0);
+                void* cst = conv_layer(li) + cofs;
+                ConvGramArgs cg{xbc_pre, proj, w.conv1d_w, w.conv1d_b, t0 ? cst : nullptr, t0 ? nullptr : cst};
+                s.gram_ready = conv_gram_takes(s, cg, K);
                 if (e == hipSuccess)
-                    e = launch_conv1d(strm, xbc_pre, proj, w.conv1d_w, w.conv1d_b, xba, xbc, nb, L, xbc, K,
-                                      act, true, t0 ? conv_layer(li) + cofs : nullptr);
-                if (e == hipSuccess)
-                    e = launch_conv1d_seed(strm, xbc_pre, proj, conv_layer(li) + cofs, nb, L, xbc, K, act);
+                    e = s.gram_ready ? launch_conv_gram(strm, s, cg)
+                                     : launch_conv1d(strm, xbc_pre, proj, w.conv1d_w, w.conv1d_b, xba, xbc, nb, L,
+                                                     xbc, K, act, true, cg.hist);
+                if (e == hipSuccess && !(s.gram_ready && cg.state))
+                    e = launch_conv1d_seed(strm, xbc_pre, proj, cst, nb, L, xbc, K, act);
                 if (e == hipSuccess) {
                     e = launch_ssd_chunked(strm, s);
                     if (e == hipSuccess && gparts)

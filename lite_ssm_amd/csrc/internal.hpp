@@ -292,12 +292,30 @@ struct SsdArgs {
     // z already holds r(silu(z)) (the projection's GEMM applied it), so
     // g = r(z r(y)); the fused gate is taken only then
     bool z_silu = false;
+    // gram already holds the tiles (launch_conv_gram)
+    bool gram_ready = false;
 };
 hipError_t launch_ssd_step(hipStream_t s, const SsdArgs& a);
 // Partials per row a decode step with SsdArgs::yfrag writes (H P / 32), or 0
 // when it cannot.
 uint32_t ssd_step_parts(uint32_t H, uint32_t P, uint32_t N, int act);
 hipError_t launch_ssd_chunked(hipStream_t s, const SsdArgs& a);
+// The conv of width 4 (with SiLU) that writes the scan's rows a.X | a.B | a.C,
+// its Gram tiles (a.gram; the scan then gets gram_ready) and, if state is not
+// null, the sequences' conv states [batch][channels][4], in one launch; where
+// conv_gram_takes.  x: the projection's xBC columns, row stride xs; hist as for
+// launch_conv1d (and then no state: the last rows would be written while the
+// first read it).
+struct ConvGramArgs {
+    const void* x;
+    uint32_t xs;
+    const void* w;
+    const void* bias;
+    const void* hist = nullptr;
+    void* state = nullptr;
+};
+bool conv_gram_takes(const SsdArgs& a, const ConvGramArgs& c, uint32_t K);
+hipError_t launch_conv_gram(hipStream_t s, const SsdArgs& a, const ConvGramArgs& c);
 // Partial sums of squares per row that launch_ssd_chunked writes when a.gpart
 // is set, or 0 where it cannot fuse the gate (not the MFMA walk).
 uint32_t ssd_chunked_gate_parts(const SsdArgs& a);

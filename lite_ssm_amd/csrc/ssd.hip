@@ -14,6 +14,7 @@
 #include <cstdlib>
 
 #include "common.hpp"
+#include "conv_core.hpp"
 #include "internal.hpp"
 
 namespace lssm {
@@ -342,25 +343,13 @@ template <typename T> __device__ __forceinline__ floatx4 unpack4(s4v v) {
     return r;
 }
 
-// The chunks' Gram tiles G[t][j] = C_t . B_j (fp32, t, j < 64), which depend
-// only on the sequence, the chunk and the group: computed once here and read
-// by every head of the group (and P slice) in ssd_chunk_mfma_kernel instead of
-// being recomputed there.  Block (chunk, group, sequence), four waves; the ten
-// tiles with J <= T (16-token blocks) only, on the same MFMA with the same
-// operands as the in-kernel computation, so the values are identical.  The
-// operands are read straight from global memory: both have k = n contiguous.
-// Tokens past the end of the last chunk re-read token t0 (their entries are
-// masked by the scan).
+// A chunk's Gram tile G[t][j] = C_t . B_j (fp32, t, j < 64) by four waves: the
+// ten 16 x 16 tiles with J <= T only.  Tokens past the chunk's end (tl tokens)
+// re-read token 0 (their entries are masked by the scan).
 template <typename T>
-__global__ __launch_bounds__(256) void ssd_gram_kernel(SsdArgs a) {
-    const uint32_t c = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
-    const uint32_t L = a.L, nch = (L + CQ - 1) / CQ, t0 = c * CQ;
-    const uint32_t tl = min((uint32_t)CQ, L - t0);
-    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+__device__ __forceinline__ void gram_tiles(const T* Bv, uint32_t bs, const T* Cv, uint32_t cs, uint32_t tl, int w,
+                                           int lane, float* out) {
     const int li = lane % 16, lq = lane / 16;
-    const T* Bv = (const T*)a.B + ((size_t)b * L + t0) * a.b_stride + (size_t)g * CN;
-    const T* Cv = (const T*)a.C + ((size_t)b * L + t0) * a.c_stride + (size_t)g * CN;
-    float* out = a.gram + (((size_t)b * nch + c) * a.G + g) * (CQ * CQ);
     // (J, T) of the ten lower tiles, 2 + 2 bits each
     constexpr uint64_t JT = 0x0ull | 0x4ull << 4 | 0x5ull << 8 | 0x8ull << 12 | 0x9ull << 16 | 0xAull << 20 |
                             0xCull << 24 | 0xDull << 28 | 0xEull << 32 | 0xFull << 36;
@@ -368,8 +357,8 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(SsdArgs a) {
         const int jt = (int)(JT >> (4 * kt)) & 15;
         const int J = jt & 3, Tt = jt >> 2;
         const uint32_t j = 16 * J + li, t = 16 * Tt + li;
-        const T* br = Bv + (size_t)(j < tl ? j : 0) * a.b_stride + 8 * lq;
-        const T* cr = Cv + (size_t)(t < tl ? t : 0) * a.c_stride + 8 * lq;
+        const T* br = Bv + (size_t)(j < tl ? j : 0) * bs + 8 * lq;
+        const T* cr = Cv + (size_t)(t < tl ? t : 0) * cs + 8 * lq;
         floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ks = 0; ks < CN / 32; ++ks)
@@ -377,6 +366,69 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(SsdArgs a) {
         // acc[r] = B_{16J + 4lq + r} . C_t  ->  G[t][16J + 4lq .. + 3]
         *reinterpret_cast<floatx4*>(out + (size_t)t * CQ + 16 * J + 4 * lq) = acc;
     }
+}
+
+// The chunks' Gram tiles, which depend only on the sequence, the chunk and the
+// group: computed once here (or by conv_gram_kernel) and read by every head of
+// the group (and P slice) in ssd_chunk_mfma_kernel instead of being recomputed
+// there, on the same MFMA with the same operands, so the values are identical.
+// Block (chunk, group, sequence); the operands are read straight from global
+// memory: both have k = n contiguous.
+template <typename T>
+__global__ __launch_bounds__(256) void ssd_gram_kernel(SsdArgs a) {
+    const uint32_t c = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    const uint32_t L = a.L, nch = (L + CQ - 1) / CQ, t0 = c * CQ;
+    gram_tiles<T>((const T*)a.B + ((size_t)b * L + t0) * a.b_stride + (size_t)g * CN, a.b_stride,
+                  (const T*)a.C + ((size_t)b * L + t0) * a.c_stride + (size_t)g * CN, a.c_stride,
+                  min((uint32_t)CQ, L - t0), (int)(threadIdx.x / WAVE), (int)(threadIdx.x % WAVE),
+                  a.gram + (((size_t)b * nch + c) * a.G + g) * (CQ * CQ));
+}
+
+constexpr int CONV_GRAM_CT = 4;
+
+// The prefill's conv, conv state and Gram tiles in one launch: a short prompt
+// spends most of these in launches (37 tokens of the 130M model: conv 6.4, state
+// 2.8, Gram 4.2 us; the whole 24-layer prefill 1.19 -> 0.96 ms with this and four
+// tokens a thread; 700 tokens of four 2.7B layers 651 -> 626 us).  Blocks 0 .. nch G - 1 take a chunk's B and C channels of a
+// group: thread (token eighth, 16-byte piece) convolves 8 tokens into memory and
+// LDS, then the block's waves multiply the rounded values as ssd_gram_kernel
+// does.  The other blocks take the x channels, four tokens a thread (a wave's
+// chain grows with the tokens; conv1d's 16 read less but want a full chip).
+template <typename T>
+__global__ __launch_bounds__(256, 4) void conv_gram_kernel(SsdArgs a, ConvGramArgs cv) {
+    __shared__ __attribute__((aligned(16))) T S[2][CQ * SPAD];    // B, C
+    const uint32_t L = a.L, nch = (L + CQ - 1) / CQ, ng = nch * a.G;
+    const uint32_t D1 = a.H * a.P, D = D1 + 2 * a.G * CN, b = blockIdx.y;
+    const T* x = (const T*)cv.x + (size_t)b * L * cv.xs;
+    const T* bias = (const T*)cv.bias;
+    T* y = const_cast<T*>((const T*)a.X) + (size_t)b * L * a.x_stride;
+    T* state = cv.state ? (T*)cv.state + (size_t)b * D * 4 : nullptr;
+    auto run = [&](auto ct, uint32_t d0, uint32_t t0, T* lds) {
+        constexpr int N = decltype(ct)::value;
+        v4u win[N + 3];
+        conv_window<T, N>(x + d0, cv.xs, t0, L, cv.hist ? (const T*)cv.hist + (size_t)d0 * 4 : nullptr, win);
+        conv_rows<T, N, true>(win, (const T*)cv.w + (size_t)d0 * 4, bias ? bias + d0 : nullptr, [&](int i, v4u o) {
+            if (t0 + i < L) *reinterpret_cast<v4u*>(y + (size_t)(t0 + i) * a.x_stride + d0) = o;
+            if (lds) *reinterpret_cast<v4u*>(lds + i * SPAD) = o;
+        });
+        if (state) conv_seed<T, N>(win, t0, L, state + (size_t)d0 * 4);
+    };
+    constexpr int CT = CONV_GRAM_CT;
+    if (blockIdx.x >= ng) {
+        const uint32_t item = (blockIdx.x - ng) * 256 + threadIdx.x, nd = D1 / 8;
+        const uint32_t t0 = item / nd * CT;
+        if (t0 < L) run(std::integral_constant<int, CT>{}, item % nd * 8, t0, nullptr);
+        return;
+    }
+    const uint32_t c = blockIdx.x % nch, g = blockIdx.x / nch, tc = c * CQ;
+    const uint32_t tl = min((uint32_t)CQ, L - tc);
+    {
+        const uint32_t pc = threadIdx.x % 32, ts = threadIdx.x / 32 * 8, m = pc / 16, n = pc % 16 * 8;
+        run(std::integral_constant<int, 8>{}, D1 + (m * a.G + g) * CN + n, tc + ts, S[m] + ts * SPAD + n);
+    }
+    __syncthreads();
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    gram_tiles<T>(S[0], SPAD, S[1], SPAD, tl, w, lane, a.gram + (((size_t)b * nch + c) * a.G + g) * (CQ * CQ));
 }
 
 // SPL = 2: two waves per 16-column slice.  Wave (slice cs, half hh) computes
@@ -1297,6 +1349,34 @@ hipError_t launch_rms_from_parts(hipStream_t s, const float* part, uint32_t npar
     return hipGetLastError();
 }
 
+// blocks of a sequence's x channels with ct tokens a thread
+uint32_t conv_gram_blocks(const SsdArgs& a, uint32_t ct) {
+    return (uint32_t)(((uint64_t)(a.H * a.P / 8) * ((a.L + ct - 1) / ct) + 255) / 256);
+}
+
+bool conv_gram_takes(const SsdArgs& a, const ConvGramArgs& c, uint32_t K) {
+    if (a.batch == 0 || a.L == 0 || !a.gram || !mfma_ok(a) || K != 4 || (a.H * a.P) % 8 != 0) return false;
+    if (c.hist && (c.state || a.batch != 1)) return false;
+    // (long prompts fill the chip with 16 tokens a thread: 16384 rows of the 2.7B
+    // model through this kernel with 16 took 0.75 ms longer over four layers, two
+    // waves a SIMD instead of three)
+    if ((uint64_t)conv_gram_blocks(a, 16) * a.batch >= 2 * num_cus()) return false;
+    const uint32_t D1 = a.H * a.P;
+    const char* y = (const char*)a.X;
+    if (a.B != y + (size_t)D1 * 2 || a.C != y + (size_t)(D1 + a.G * CN) * 2) return false;
+    if (a.b_stride != a.x_stride || a.c_stride != a.x_stride || a.x_stride < D1 + 2 * a.G * CN || c.xs % 8 != 0) return false;
+    for (const void* p : {c.x, c.w, c.bias, (const void*)c.state})
+        if ((uintptr_t)p % 16 != 0) return false;
+    return true;
+}
+
+hipError_t launch_conv_gram(hipStream_t s, const SsdArgs& a, const ConvGramArgs& c) {
+    const dim3 grid((a.L + CQ - 1) / CQ * a.G + conv_gram_blocks(a, CONV_GRAM_CT), a.batch);
+    if (a.act == LSSM_F16) conv_gram_kernel<f16><<<grid, 256, 0, s>>>(a, c);
+    else conv_gram_kernel<bf16><<<grid, 256, 0, s>>>(a, c);
+    return hipGetLastError();
+}
+
 hipError_t launch_ssd_chunked(hipStream_t s, const SsdArgs& a0) {
     if (a0.batch == 0 || a0.H == 0 || a0.L == 0) return hipSuccess;
     SsdArgs a = a0;
@@ -1319,7 +1399,7 @@ hipError_t launch_ssd_chunked(hipStream_t s, const SsdArgs& a0) {
         const bool gp = a.gram != nullptr;
         auto go = [&](auto tag) {
             using T = decltype(tag);
-            if (gp) {
+            if (gp && !a.gram_ready) {
                 const dim3 gg(nch, a.G, a.batch);
                 ssd_gram_kernel<T><<<gg, 256, 0, s>>>(a);
             }
