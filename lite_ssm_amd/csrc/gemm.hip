@@ -578,7 +578,7 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Skinny GEMM for decode batches (5 <= M <= 64): the weights are streamed once.
+// Skinny GEMM for few rows (up to 48): the weights are streamed once.
 // A block covers 16 rows of W; its KS waves split K into slices of UPW units,
 // and the slices are summed in LDS.  A lane loads 16 bytes of one W row per
 // unit (int4: 32 k, int8: 16, dense: 8) and dequantizes them (to r(q s), GEMM
@@ -586,7 +586,10 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
 // unit takes, in lane group q = lane / 16, the k = unit + KPL q + 8 s .. + 8
 // (the k order inside an MFMA is free as long as both operands follow it), so
 // x is read as matching 16-byte runs of its rows (L2-resident, shared by all
-// blocks).  All loads of a wave are issued before its first MFMA.
+// blocks).  All loads of a wave are issued before its first MFMA, the residual
+// and the row scale of the wave's tile among them; the slices' sums and the
+// epilogue are spread over a wave per 16 rows (one wave for all, with its loads
+// behind the sums: 32 x 768 x 1536 int8 8.4 us, now 7.0).
 // ---------------------------------------------------------------------------
 template <int FMT> struct SkUnit {
     static constexpr int KPL = FMT == LSSM_W_DENSE ? 8 : (FMT == LSSM_W_Q8_G32 ? 16 : 32);
@@ -607,14 +610,14 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
     using SU = SkUnit<FMT>;
     constexpr int KPL = SU::KPL, U = SU::U, STEPS = SU::STEPS;
     constexpr uint32_t GS = FMT == LSSM_W_Q4_G64 ? 64 : 32;
-    __shared__ floatx4 red[SK_MAXW - 1][MT][64];
+    __shared__ floatx4 red[SK_MAXW][MT][64];
 
     const int lane = threadIdx.x % WAVE;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int KS = blockDim.x / WAVE;
     const int li = lane % 16, lq = lane / 16;
     const uint32_t n0 = blockIdx.x * 16;
-    const uint32_t K = a.K, kb = w * (UPW * U);
+    const uint32_t K = a.K, KS = K / (UPW * U);
+    const uint32_t kb = min((uint32_t)w, KS - 1) * (UPW * U);   // (waves past KS only finish a tile)
     const uint32_t n = min(n0 + li, a.N - 1);
 
     const char* wrow;
@@ -641,6 +644,17 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int st = 0; st < STEPS; ++st) r[uu].x[mt][st] = *reinterpret_cast<const u32x4*>(xrow[mt] + k + 8 * st);
+    }
+    // wave mt finishes row tile mt: its scale and residual come with the rest
+    const uint32_t mo = 16u * w + li, no = n0 + 4 * lq;
+    const bool own = w < MT && mo < a.M;
+    T res[4];
+    float rs = 1.0f;
+    if (own) {
+        if (a.row_scale) rs = a.row_scale[mo];
+        if (EPI == LSSM_EPI_ADD)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) res[rr] = ((const T*)a.res)[(size_t)mo * a.y_stride + min(no + rr, a.N - 1)];
     }
     // all loads in flight before the first MFMA (when they fit the registers:
     // 16-wave blocks leave 128 VGPRs)
@@ -675,34 +689,26 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
             for (int mt = 0; mt < MT; ++mt) acc[mt] = mma16x32<T>(af[st], r[uu].x[mt][st], acc[mt]);
     }
 
-    // sum the K slices; wave 0 stores.  D element r of lane l: row
-    // 4 (l / 16) + r (W row n0 + .), column l % 16 (x row 16 mt + .).
-    if (w > 0) {
+    // sum the K slices in order; waves 0 .. MT - 1 a row tile each (the launcher
+    // gives the block MT waves).  D element r of lane l: row 4 (l / 16) + r (W row
+    // n0 + .), column l % 16 (x row 16 mt + .).
+    if (w < (int)KS) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) red[w - 1][mt][lane] = acc[mt];
+        for (int mt = 0; mt < MT; ++mt) red[w][mt][lane] = acc[mt];
     }
     __syncthreads();
-    if (w != 0) return;
+    if (!own) return;
     T* Y = (T*)a.y;
-    const T* R = (const T*)a.res;
+    floatx4 v = red[0][w][lane];
+    for (uint32_t q = 1; q < KS; ++q) v += red[q][w][lane];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        floatx4 v = acc[mt];
-        for (int q = 0; q < KS - 1; ++q) v += red[q][mt][lane];
-        const uint32_t m = 16 * mt + li;
-        if (m >= a.M) continue;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const uint32_t nn = n0 + 4 * lq + rr;
-            if (nn >= a.N) continue;
-            const size_t yi = (size_t)m * a.y_stride + nn;
-            float o = v[rr];
-            if (a.row_scale) o *= a.row_scale[m];
-            if (nn < a.silu_cols) o = silu_fast(o);
-            if (EPI == LSSM_EPI_SILU) o = silu_f(o);
-            if (EPI == LSSM_EPI_ADD) o = to_f(R[yi]) + rnd<T>(o);
-            Y[yi] = from_f<T>(o);
-        }
+    for (int rr = 0; rr < 4; ++rr) {
+        if (no + rr >= a.N) continue;
+        float o = v[rr] * rs;
+        if (no + rr < a.silu_cols) o = silu_fast(o);
+        if (EPI == LSSM_EPI_SILU) o = silu_f(o);
+        if (EPI == LSSM_EPI_ADD) o = to_f(res[rr]) + rnd<T>(o);
+        Y[(size_t)mo * a.y_stride + no + rr] = from_f<T>(o);
     }
 }
 
@@ -750,7 +756,7 @@ __global__ void gemm_simple_kernel(GemmArgs a) {
 template <int FMT, typename T, int MT, int UPW>
 hipError_t go_skinny(hipStream_t s, const GemmArgs& a) {
     const dim3 grid((a.N + 15) / 16);
-    const dim3 block(64 * (a.K / (UPW * SkUnit<FMT>::U)));
+    const dim3 block(64 * std::max<uint32_t>(MT, a.K / (UPW * SkUnit<FMT>::U)));
     switch (a.epi) {
         case LSSM_EPI_SILU: gemm_skinny_kernel<FMT, T, LSSM_EPI_SILU, MT, UPW><<<grid, block, 0, s>>>(a); break;
         case LSSM_EPI_ADD: gemm_skinny_kernel<FMT, T, LSSM_EPI_ADD, MT, UPW><<<grid, block, 0, s>>>(a); break;
@@ -817,11 +823,10 @@ inline bool gemm_takes_mid(const GemmArgs& a) {
 
 // Units per wave of the skinny kernel for a call, 0 where it does not take it:
 // few rows, weights streamed once.  Every block reads all of x, so past 16 rows
-// only while that is small: 37 x 10576 x 2560 int4 26.2 us against 15.2 in
-// gemm_mid, 32 x 768 x 1536 int8 8.4 against 9.2, 37 x 3352 x 768 int8 6.6
-// against 7.5 (64 rows: 7.8 against 7.6).
+// only while that is small (us, here / gemm_mid): 37 x 10576 x 2560 int4 26.2 /
+// 15.2, 32 x 768 x 1536 int8 7.0 / 9.2, 37 x 3352 x 768 int8 6.2 / 7.5.
 template <int FMT> int skinny_takes(const GemmArgs& a) {
-    if (a.M > 48 || (a.M > 32 && a.K > 1024) || (a.M > 16 && a.K > 2048)) return 0;
+    if (a.M > 48 || (a.M > 16 && a.K > 2048)) return 0;
     return skinny_upw<FMT>(a.K, (int)(a.M + 15) / 16);
 }
 
