@@ -779,7 +779,9 @@ template <int FMT> int skinny_upw(uint32_t K, int mt) {
 
 template <int FMT, typename T, int MT>
 hipError_t go_skinny_mt(hipStream_t s, const GemmArgs& a, int upw) {
-    if (upw == 4) return go_skinny<FMT, T, MT, 4>(s, a);
+    // (quantized weights past 16 rows, K <= 2048: one or two units always do)
+    if constexpr (MT == 1 || FMT == LSSM_W_DENSE)
+        if (upw == 4) return go_skinny<FMT, T, MT, 4>(s, a);
     if (upw == 2) return go_skinny<FMT, T, MT, 2>(s, a);
     return go_skinny<FMT, T, MT, 1>(s, a);
 }
