@@ -394,8 +394,11 @@ constexpr int CONV_GRAM_CT = 4;
 // LDS, then the block's waves multiply the rounded values as ssd_gram_kernel
 // does.  The other blocks take the x channels, four tokens a thread (a wave's
 // chain grows with the tokens; conv1d's 16 read less but want a full chip).
+// Four waves a SIMD, but three for f16, which spills 14 registers at four: 130M
+// prefill of 37 tokens 906 -> 885 us, of 500 1550 -> 1518, of 3000 and 1400 tokens
+// of the 2.7B the same.
 template <typename T>
-__global__ __launch_bounds__(256, 4) void conv_gram_kernel(SsdArgs a, ConvGramArgs cv) {
+__global__ __launch_bounds__(256, __is_same(T, f16) ? 3 : 4) void conv_gram_kernel(SsdArgs a, ConvGramArgs cv) {
     __shared__ __attribute__((aligned(16))) T S[2][CQ * SPAD];    // B, C
     const uint32_t L = a.L, nch = (L + CQ - 1) / CQ, ng = nch * a.G;
     const uint32_t D1 = a.H * a.P, D = D1 + 2 * a.G * CN, b = blockIdx.y;
