@@ -33,6 +33,9 @@ template <int FMT, int BM, int BN> struct MidShape {
 };
 
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+template <int VM, int LGKM> __device__ __forceinline__ void wait_vm_lds() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(%1)" ::"n"(VM), "n"(LGKM) : "memory");
+}
 
 template <int FMT, typename T, int BM, int BN>
 __global__ __launch_bounds__(64 * (4 + MidShape<FMT, BM, BN>::PROD)) void gemm_mid_kernel(GemmArgs a) {
@@ -227,7 +230,11 @@ __global__ __launch_bounds__(64 * (4 + MidShape<FMT, BM, BN>::PROD)) void gemm_m
         xs = xn;
         bs = bn;
         xd = xd + 1 == XS ? 0 : xd + 1;
-        wait_vm<XJ * (XS - 3)>();                              // stage kt + 2 of X landed
+        // stage kt + 2 of X landed, and this wave's reads of stage kt done:
+        // behind the barrier its slot is filled again.  (LDS reads complete in
+        // order, and only those of the last three sub-steps, all of stage kt +
+        // 1, may be outstanding; the first sub-step's DMA keeps them behind.)
+        wait_vm_lds<XJ * (XS - 3), 3 * (MI + NI)>();
         barrier();
     }
     wait_vm<0>();
