@@ -446,6 +446,7 @@ GemmMidPlan gemm_mid_plan(const GemmArgs& a) {
         uint32_t ends, q, q_min, d, d_min;
     };
     for (const Tile& t : {Tile{128, 128, 500, 57, 54, 57, 40}, Tile{128, 64, 300, 45, 37, 35, 27}, Tile{64, 64, 250, 27, 27, 21, 21}}) {
+        if (((uint64_t)a.M + t.bm - 1) / t.bm > 65535) continue;      // (grid.y)
         const uint64_t tiles = (uint64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn);
         const bool pair = !dense && t.bm == 64;
         for (uint32_t S : {1u, 2u, 3u, 4u, 5u, 6u, 8u}) {
