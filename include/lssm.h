@@ -26,6 +26,19 @@
  * error check), like the reference's one-shot command buffer (ops.mm:131-148).
  * Inside lssm_begin_batch / lssm_commit_and_wait ops only enqueue
  * (ops.mm:82-112).
+ *
+ * HIP graphs: inside a batch, ops may be enqueued while the context's stream is
+ * being captured.  The captured launches hold the caller's buffers only, so the
+ * graphs may be replayed on any stream, beside other work of the context and
+ * after it is destroyed.  Exceptions: lssm_ssd_chunked holds workspaces of the
+ * context (replays must be ordered with its other scans, and the context must
+ * outlive the graph); lssm_embed and the fused batch-1 entries hold its status
+ * word (it must outlive the graph); and what the entries below state.
+ * Captured, lssm_linear runs with K unsplit where it otherwise splits it over
+ * several blocks (the same products, summed in another order), and
+ * lssm_norm_linear_decode and lssm_inproj_decode normalise their rows again in
+ * each block instead of once (the same results; a wide dense weight of more
+ * than four rows, another order of sums).
  */
 #ifndef LSSM_H
 #define LSSM_H

@@ -34,17 +34,29 @@ bool gemm_ok(const void* x, uint32_t x_stride, const void* w, uint32_t K, int ac
     return act != LSSM_F32 && K % 64 == 0 && x_stride % 8 == 0 && al16(x) && al16(w);
 }
 
+// Whether a call may pass data between its launches in the context's memory:
+// not while the stream is captured (or its state cannot be asked for).
+bool scratch_ok(const lssm_ctx* ctx) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cap == hipStreamCaptureStatusNone;
+}
+
 // Decode batches whose x is packed once into the context's buffer for the
-// batched GEMV.
+// batched GEMV (captured: normalised by each of its blocks, the same outputs).
 bool pack_rows_ok(const lssm_ctx* ctx, const GemvArgs& g) {
     return g.norm_w && ctx->xpack && gemv_rows_pays(g.M, g.N, g.K, g.wfmt, g.act) && al16(g.x) &&
            al16(g.norm_w) && al16(g.w) && (g.wfmt == LSSM_W_DENSE || (uintptr_t)g.s % 4 == 0) && g.x_stride % 8 == 0;
 }
 hipError_t pack_rows(lssm_ctx* ctx, GemvArgs& g) {
+    g.xrows = true;
+    if (!scratch_ok(ctx)) return hipSuccess;
     const hipError_t e = launch_mma_pack(ctx->stream, g.x, g.x_stride, g.norm_w, g.eps, g.M, g.K, g.wfmt, g.act,
                                          ctx->xpack);
     g.xpack = ctx->xpack;
-    g.xrows = true;
     return e;
 }
 
@@ -81,16 +93,11 @@ int linear_core(lssm_ctx* ctx, const void* x, uint32_t xs, const void* w, const 
     } else if (!gemv && gemm_ok(x, xs, w, K, act)) {
         GemmArgs g{x, xs, w, s, y, ys, res, M, N, K, wfmt, act, epi, 1};
         std::unique_lock<std::mutex> lk(ctx->scratch_mu, std::defer_lock);
-        const bool split = gemm_wants_ws(g);
+        const bool split = gemm_wants_ws(g) && scratch_ok(ctx);
         if (split) lk.lock();
-        if (split && !ctx->gemm_ws) {
-            // (not while the stream is captured: the call then runs unsplit)
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-                hipMalloc((void**)&ctx->gemm_ws, GEMM_WS_FLOATS * sizeof(float)) != hipSuccess) {
-                ctx->gemm_ws = nullptr;
-                (void)hipGetLastError();
-            }
+        if (split && !ctx->gemm_ws && hipMalloc((void**)&ctx->gemm_ws, GEMM_WS_FLOATS * sizeof(float)) != hipSuccess) {
+            ctx->gemm_ws = nullptr;
+            (void)hipGetLastError();
         }
         if (split && ctx->gemm_ws) {
             g.ws = ctx->gemm_ws;
@@ -155,7 +162,11 @@ int lssm_norm_linear_decode(lssm_ctx* ctx, const void* x, const void* norm_w, fl
     GemvArgs g{x, K, w, w_scales, y, N, residual, norm_w, eps, rows, N, K, wfmt, act, epi};
     hipError_t e;
     std::unique_lock<std::mutex> lk(ctx->scratch_mu);
-    if (rows > 4 && dense_head_gemm(N, K, wfmt, act) && al16(x) && al16(norm_w)) {
+    const bool head = rows > 4 && dense_head_gemm(N, K, wfmt, act) && al16(x) && al16(norm_w);
+    if (head && !scratch_ok(ctx)) {
+        g.xrows = gemv_rows_takes(rows, N, K, wfmt, act);
+        e = launch_gemv(ctx->stream, g);
+    } else if (head) {
         // an lm_head: norm launch, then the tiled GEMM (dense: one rule)
         e = launch_rmsnorm(ctx->stream, x, K, norm_w, ctx->xpack, K, rows, K, eps, act);
         GemmArgs m{ctx->xpack, K, w, nullptr, y, N, residual, rows, N, K, wfmt, act, epi, 1};

@@ -1188,10 +1188,7 @@ __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_s
         xv = reinterpret_cast<const u32x4*>(x + (size_t)m * x_stride)[cc];
         nv = reinterpret_cast<const u32x4*>(nw)[cc];
     }
-    float q = dot2(xv[0], xv[0], 0.0f, T{});
-    q = dot2(xv[1], xv[1], q, T{});
-    q = dot2(xv[2], xv[2], q, T{});
-    q = dot2(xv[3], xv[3], q, T{});
+    float q = octet_squares<T>(xv);
     // block sum in a fixed order: waves, then the wave sums in wave order
     q = wave_sum(q);
     const uint32_t nwv = blockDim.x / WAVE;
@@ -1199,25 +1196,12 @@ __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_s
     __syncthreads();
     float t = 0.0f;
     for (uint32_t i = 0; i < nwv; ++i) t += red[i];
-    const float rr = 1.0f / sqrtf(t / (float)K + eps);
+    const float rr = row_inv_rms(t, K, eps);
     // part: x w without 1 / rms, the sum of squares to part[4 m]
     const bool raw = part != nullptr;
     if (raw && threadIdx.x < 4) part[4 * m + threadIdx.x] = threadIdx.x == 0 ? t : 0.0f;
     if (!live) return;
-    const float sc = raw ? 1.0f : rr;
-    float v[8];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        v[2 * e] = lo_f<T>(xv[e]) * lo_f<T>(nv[e]) * sc;
-        v[2 * e + 1] = hi_f<T>(xv[e]) * hi_f<T>(nv[e]) * sc;
-    }
-    u32x4 pk;
-#pragma unroll
-    for (int qq = 0; qq < 4; ++qq) {
-        int pa, pb;
-        octet_pos<FMT, T>(qq, pa, pb);
-        pk[qq] = pack2<T>(v[pa], v[pb]);
-    }
+    const u32x4 pk = octet_scaled<FMT, T>(xv, nv, raw ? 1.0f : rr);
     // octet cc of quad qa: chunk ch, pair offset 4 p4 of the chunk; k-slice sl
     // and lane group lg with mma_slice_pos(sl, lg) = (ch, 4 p4)
     using P = Mma<FMT, T>;

@@ -107,6 +107,36 @@ template <typename T> __device__ __forceinline__ floatx4 mfma16(u32x4 a, u32x4 b
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
 }
 
+// RMSNorm of x for these kernels (norm.metal:52-79), the same wherever a row is
+// normalised: the squares of an octet (summed over the lanes by wave_sum, over
+// the runs of 64 octets in order), 1 / rms of a row of K with that sum, and
+// r(x w scale) of an octet in the unpack's pair order.
+template <typename T> __device__ __forceinline__ float octet_squares(u32x4 xv) {
+    float q = dot2(xv[0], xv[0], 0.0f, T{});
+    q = dot2(xv[1], xv[1], q, T{});
+    q = dot2(xv[2], xv[2], q, T{});
+    return dot2(xv[3], xv[3], q, T{});
+}
+__device__ __forceinline__ float row_inv_rms(float squares, uint32_t K, float eps) {
+    return 1.0f / sqrtf(squares / (float)K + eps);
+}
+template <int FMT, typename T> __device__ __forceinline__ u32x4 octet_scaled(u32x4 xv, u32x4 nv, float scale) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[2 * e] = lo_f<T>(xv[e]) * lo_f<T>(nv[e]) * scale;
+        v[2 * e + 1] = hi_f<T>(xv[e]) * hi_f<T>(nv[e]) * scale;
+    }
+    u32x4 pk;
+#pragma unroll
+    for (int qq = 0; qq < 4; ++qq) {
+        int pa, pb;
+        octet_pos<FMT, T>(qq, pa, pb);
+        pk[qq] = pack2<T>(v[pa], v[pb]);
+    }
+    return pk;
+}
+
 // Every format, for the kernels that take them all.
 template <typename T, class F> bool all_fmt(int wfmt, F&& f) {
     if constexpr (__is_same(T, float)) {

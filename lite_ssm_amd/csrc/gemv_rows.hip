@@ -29,14 +29,65 @@ namespace {
 constexpr int GR_W = 8;                          // waves per block: the K split
 constexpr int GR_D = 2;                          // quads in flight per wave
 
+template <int FMT, typename T> constexpr int scale_dwords() {   // per tile and quad
+    return Mma<FMT, T>::G > 0 ? Mma<FMT, T>::GPQ / 2 : 1;
+}
+
+// acc += the products of one quad: w as loaded, s its scales, x in fragment order.
+template <int FMT, typename T, int CT, int RT>
+__device__ __forceinline__ void rows_quad(const u32x4 (&w)[CT], const uint32_t (&s)[CT][scale_dwords<FMT, T>()],
+                                          const u32x4 (&x)[RT][Mma<FMT, T>::SPQ], floatx4 (&acc)[RT][CT]) {
+    using P = Mma<FMT, T>;
+    constexpr int GPQ = P::GPQ, SPG = P::SPG;
+    u32x4 wq[CT];
+#pragma unroll
+    for (int t = 0; t < CT; ++t) wq[t] = mma_swap<FMT>(w[t]);
+    if constexpr (P::G == 0) {
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[rt][t] = mfma16<T>(x[rt][0], wq[t], acc[rt][t]);
+    } else {
+#pragma unroll
+        for (int g = 0; g < GPQ; ++g) {
+            floatx4 c0[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                c0[rt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (P::BIAS) {
+                    constexpr uint32_t M136 = 0xC308C308u;             // bf16 (-136, -136)
+#pragma unroll
+                    for (int e = 0; e < SPG; ++e)
+                        c0[rt] = mfma16<T>(x[rt][g * SPG + e], u32x4{M136, M136, M136, M136}, c0[rt]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                u32x4 u[SPG];
+#pragma unroll
+                for (int e = 0; e < SPG; ++e) u[e] = unpack_slice<FMT, T>(wq[t], g * SPG + e);
+                const uint32_t sw = s[t][g / 2];
+                const float sc = fp16_bits_to_f((uint16_t)((g & 1) ? sw >> 16 : sw & 0xFFFFu));
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    floatx4 d = c0[rt];
+#pragma unroll
+                    for (int e = 0; e < SPG; ++e) d = mfma16<T>(x[rt][g * SPG + e], u[e], d);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[rt][t][i] = __builtin_fmaf(sc, d[i], acc[rt][t][i]);
+                }
+            }
+        }
+    }
+}
+
 template <int FMT, typename T, int CT, int RT, class Epi>
 __global__ __launch_bounds__(64 * GR_W) void gemv_rows_kernel(GemvCore c, Epi epi, uint32_t M, uint32_t qpw) {
     using P = Mma<FMT, T>;
     using F = Fmt<FMT, T>;
-    constexpr int SPQ = P::SPQ, GPQ = P::GPQ, SPG = P::SPG;
-    constexpr bool BIAS = P::BIAS;
+    constexpr int SPQ = P::SPQ;
     constexpr int D = GR_D;
-    constexpr int SW = P::G > 0 ? GPQ / 2 : 1;                 // scale dwords per tile and quad
+    constexpr int SW = scale_dwords<FMT, T>();
     extern __shared__ __attribute__((aligned(16))) uint32_t mm_lds[];
 
     const uint32_t K = c.K, N = c.N;
@@ -84,48 +135,7 @@ __global__ __launch_bounds__(64 * GR_W) void gemv_rows_kernel(GemvCore c, Epi ep
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int t = 0; t < CT; ++t) acc[rt][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto compute = [&](const Slot& r) {
-        u32x4 wq[CT];
-#pragma unroll
-        for (int t = 0; t < CT; ++t) wq[t] = mma_swap<FMT>(r.w[t]);
-        if constexpr (P::G == 0) {
-#pragma unroll
-            for (int t = 0; t < CT; ++t)
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) acc[rt][t] = mfma16<T>(r.x[rt][0], wq[t], acc[rt][t]);
-        } else {
-#pragma unroll
-            for (int g = 0; g < GPQ; ++g) {
-                floatx4 c0[RT];
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) {
-                    c0[rt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (BIAS) {
-                        constexpr uint32_t M136 = 0xC308C308u;             // bf16 (-136, -136)
-#pragma unroll
-                        for (int e = 0; e < SPG; ++e)
-                            c0[rt] = mfma16<T>(r.x[rt][g * SPG + e], u32x4{M136, M136, M136, M136}, c0[rt]);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < CT; ++t) {
-                    u32x4 u[SPG];
-#pragma unroll
-                    for (int e = 0; e < SPG; ++e) u[e] = unpack_slice<FMT, T>(wq[t], g * SPG + e);
-                    const uint32_t sw = r.s[t][g / 2];
-                    const float sc = fp16_bits_to_f((uint16_t)((g & 1) ? sw >> 16 : sw & 0xFFFFu));
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) {
-                        floatx4 d = c0[rt];
-#pragma unroll
-                        for (int e = 0; e < SPG; ++e) d = mfma16<T>(r.x[rt][g * SPG + e], u[e], d);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[rt][t][i] = __builtin_fmaf(sc, d[i], acc[rt][t][i]);
-                    }
-                }
-            }
-        }
-    };
+    auto compute = [&](const Slot& r) { rows_quad<FMT, T, CT, RT>(r.w, r.s, r.x, acc); };
     constexpr uint32_t NT = 64 * GR_W, NO = RT * CT * 256;     // threads, output elements of the block
     constexpr int EPT = (NO + NT - 1) / NT;
     typename Epi::Pre pre[EPT];
@@ -184,6 +194,98 @@ __global__ __launch_bounds__(64 * GR_W) void gemv_rows_kernel(GemvCore c, Epi ep
             if (m < M && n < N && o / 256 % CT + tile0 < tiles) epi((int)m, n, v, pre[k]);
         }
     }
+}
+
+// The same product without x packed beforehand, for calls that may hold no
+// scratch memory (captured into a graph): a block takes one tile of 16 W rows
+// and one of 16 batch rows, forms the rows' 1 / rms and normalises x as it
+// loads it, in gemv_rows_kernel's K split and order of sums, so the outputs are
+// those of the packed form bit for bit.  Every block normalises all of its x.
+template <int FMT, typename T, class Epi>
+__global__ __launch_bounds__(64 * GR_W) void gemv_rows_norm_kernel(GemvCore c, Epi epi, uint32_t M, uint32_t qpw) {
+    using P = Mma<FMT, T>;
+    using F = Fmt<FMT, T>;
+    constexpr int SPQ = P::SPQ, D = GR_D, SW = scale_dwords<FMT, T>();
+    __shared__ floatx4 red[GR_W][WAVE];
+    __shared__ float inv_rms[16];
+
+    const uint32_t K = c.K, N = c.N, KO = K / 8;
+    const int lane = threadIdx.x % WAVE, li = lane % 16, lq = lane / 16;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t m0 = 16 * blockIdx.y, n0 = 16 * blockIdx.x;
+    const uint32_t quads = K / P::QK, q0 = w * qpw, q1 = min(q0 + qpw, quads);
+    epi.pin();
+
+    const T* x = static_cast<const T*>(c.x);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const u32x4* row = reinterpret_cast<const u32x4*>(x + (size_t)min(m0 + 2 * w + r, M - 1) * c.x_stride);
+        float t = 0.0f;
+        for (uint32_t i = 0; i < KO; i += WAVE) {
+            const uint32_t cc = i + lane;
+            t += wave_sum(octet_squares<T>(cc < KO ? row[cc] : u32x4{0u, 0u, 0u, 0u}));
+        }
+        if (lane == 0) inv_rms[2 * w + r] = row_inv_rms(t, K, c.eps);
+    }
+    __syncthreads();
+    const float scale = inv_rms[li];
+
+    struct Slot {
+        u32x4 w[1], x[SPQ], n[SPQ];
+        uint32_t s[1][SW];
+    };
+    Slot ring[D];
+    // (rows past the batch re-read its last, never stored; W rows likewise)
+    const T* xrow = x + (size_t)min(m0 + li, M - 1) * c.x_stride;
+    const T* nw = static_cast<const T*>(c.norm_w);
+    const size_t n = min(n0 + li, N - 1);
+    const uint8_t* wp = c.w + n * F::row_bytes(K) + 16 * lq;
+    const uint32_t* sp = P::G > 0 ? reinterpret_cast<const uint32_t*>(c.s + n * (K / (P::G > 0 ? P::G : 1))) : nullptr;
+    auto load = [&](uint32_t q, Slot& r) {
+        const uint32_t qa = min(q, quads - 1);
+        r.w[0] = *reinterpret_cast<const u32x4*>(wp + (size_t)64 * qa);
+        if constexpr (P::G > 0) {
+#pragma unroll
+            for (int i = 0; i < SW; ++i) r.s[0][i] = sp[qa * SW + i];
+        }
+#pragma unroll
+        for (int sl = 0; sl < SPQ; ++sl) {
+            int ch, po;
+            mma_slice_pos<FMT>(sl, lq, ch, po);
+            const uint32_t k = qa * P::QK + ch * P::WPC + 2 * po;
+            r.x[sl] = *reinterpret_cast<const u32x4*>(xrow + k);
+            r.n[sl] = *reinterpret_cast<const u32x4*>(nw + k);
+        }
+    };
+    floatx4 acc[1][1] = {{floatx4{0.0f, 0.0f, 0.0f, 0.0f}}};
+    auto compute = [&](const Slot& r) {
+        u32x4 xf[1][SPQ];
+#pragma unroll
+        for (int sl = 0; sl < SPQ; ++sl) xf[0][sl] = octet_scaled<FMT, T>(r.x[sl], r.n[sl], scale);
+        rows_quad<FMT, T, 1, 1>(r.w, r.s, xf, acc);
+    };
+    if (q0 < q1) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) load(q0 + d, ring[d]);
+    }
+    const uint32_t o = threadIdx.x, ol = (o % 256) / 4;         // output element of threads 0 .. 255
+    const uint32_t om = m0 + 4 * (ol / 16) + o % 4, on = n0 + ol % 16;
+    const typename Epi::Pre pre = epi.prefetch((int)min(om, M - 1), min(on, N - 1));
+    for (uint32_t q = q0; q < q1; q += D) {                     // (wave-uniform)
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (q + d < q1) compute(ring[d]);
+            load(q + D + d, ring[d]);
+        }
+    }
+    if (q0 < q1) red[w][lane] = acc[0][0];
+    __syncthreads();
+    if (o >= 256 || om >= M || on >= N) return;
+    const float* redf = reinterpret_cast<const float*>(&red[0][0]);
+    const uint32_t nw_run = (quads + qpw - 1) / qpw;            // waves with work
+    float v = 0.0f;
+    for (uint32_t ww = 0; ww < nw_run; ++ww) v += redf[ww * 256 + o];
+    epi((int)om, on, v, pre);
 }
 
 // gemv_rows launch plan.  Row tiles 1, 2 or 4.  Tiles of W per block by rounds
@@ -262,9 +364,16 @@ bool rows_call(hipStream_t s, const GemvArgs& a, const Epi& e, hipError_t& err) 
     return all_fmt<T>(a.wfmt, [&](auto tag) -> bool {
         constexpr int FMT = decltype(tag)::value;
         RowsPlan p;
-        const bool ok = c.xp && !a.xpart && !a.yfrag && (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.xpack % 16 == 0 &&
+        const bool ok = !a.xpart && !a.yfrag && (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.xpack % 16 == 0 &&
                         (FMT == LSSM_W_DENSE || (uintptr_t)a.s % 4 == 0) && rows_plan<FMT, T>(a.M, a.N, a.K, p);
-        err = ok ? rows_go<FMT, T, Epi>(s, c, e, a.M, p) : hipErrorInvalidValue;
+        if (ok && c.xp) {
+            err = rows_go<FMT, T, Epi>(s, c, e, a.M, p);
+        } else if (ok && a.norm_w && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.norm_w % 16 == 0 && a.x_stride % 8 == 0) {
+            gemv_rows_norm_kernel<FMT, T, Epi><<<dim3((a.N + 15) / 16, (a.M + 15) / 16), WAVE * GR_W, 0, s>>>(c, e, a.M, p.qpw);
+            err = hipGetLastError();
+        } else {
+            err = hipErrorInvalidValue;
+        }
         return true;
     });
 }

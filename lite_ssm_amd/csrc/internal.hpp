@@ -43,7 +43,9 @@ struct lssm_ctx {
     // x rows packed for the batched decode GEMV (lssm::GEMV_PACK_BYTES)
     void* xpack = nullptr;
     // held while a call enqueues the launches that pass gemm_ws or xpack on to
-    // each other (two threads on one context)
+    // each other (two threads on one context).  A call that is captured uses
+    // neither: its graph may be replayed beside the context's other work, on
+    // other streams and after the context.
     std::mutex scratch_mu;
 };
 
@@ -153,7 +155,8 @@ struct GemvArgs {
     // x rows as launch_mma_pack wrote them (norm_w applied), or null; used by
     // the MFMA decode GEMV, which then copies instead of normalising
     const void* xpack = nullptr;
-    // xpack is for the gemv_rows kernel, which takes the call (gemv_rows_takes)
+    // the gemv_rows kernel takes the call (gemv_rows_takes): x from xpack, or
+    // where that is null normalised by every block (norm_w; 16-byte aligned)
     bool xrows = false;
     // with xpack in fragment order: xpack holds r(x norm_w) without the
     // rows' 1 / rms, which the GEMV forms from their partial sums of squares
