@@ -47,16 +47,16 @@ bool scratch_ok(const lssm_ctx* ctx) {
 
 // Decode batches whose x is packed once into the context's buffer for the
 // batched GEMV (captured: normalised by each of its blocks, the same outputs).
-bool pack_rows_ok(const lssm_ctx* ctx, const GemvArgs& g) {
-    return g.norm_w && ctx->xpack && gemv_rows_pays(g.M, g.N, g.K, g.wfmt, g.act) && al16(g.x) &&
+bool pack_rows_ok(const GemvArgs& g) {
+    return g.norm_w && gemv_rows_pays(g.M, g.N, g.K, g.wfmt, g.act) && al16(g.x) &&
            al16(g.norm_w) && al16(g.w) && (g.wfmt == LSSM_W_DENSE || (uintptr_t)g.s % 4 == 0) && g.x_stride % 8 == 0;
 }
 hipError_t pack_rows(lssm_ctx* ctx, GemvArgs& g) {
     g.xrows = true;
     if (!scratch_ok(ctx)) return hipSuccess;
     const hipError_t e = launch_mma_pack(ctx->stream, g.x, g.x_stride, g.norm_w, g.eps, g.M, g.K, g.wfmt, g.act,
-                                         ctx->xpack);
-    g.xpack = ctx->xpack;
+                                         ctx->scratch);
+    g.xpack = ctx->scratch;
     return e;
 }
 
@@ -94,13 +94,9 @@ int linear_core(lssm_ctx* ctx, const void* x, uint32_t xs, const void* w, const 
         GemmArgs g{x, xs, w, s, y, ys, res, M, N, K, wfmt, act, epi, 1};
         std::unique_lock<std::mutex> lk(ctx->scratch_mu, std::defer_lock);
         const bool split = gemm_wants_ws(g) && scratch_ok(ctx);
-        if (split) lk.lock();
-        if (split && !ctx->gemm_ws && hipMalloc((void**)&ctx->gemm_ws, GEMM_WS_FLOATS * sizeof(float)) != hipSuccess) {
-            ctx->gemm_ws = nullptr;
-            (void)hipGetLastError();
-        }
-        if (split && ctx->gemm_ws) {
-            g.ws = ctx->gemm_ws;
+        if (split) {
+            lk.lock();
+            g.ws = static_cast<float*>(ctx->scratch);
             g.ws_floats = GEMM_WS_FLOATS;
         }
         e = launch_gemm(ctx->stream, g);   // (the lock ends with this block, before finish() waits)
@@ -168,11 +164,11 @@ int lssm_norm_linear_decode(lssm_ctx* ctx, const void* x, const void* norm_w, fl
         e = launch_gemv(ctx->stream, g);
     } else if (head) {
         // an lm_head: norm launch, then the tiled GEMM (dense: one rule)
-        e = launch_rmsnorm(ctx->stream, x, K, norm_w, ctx->xpack, K, rows, K, eps, act);
-        GemmArgs m{ctx->xpack, K, w, nullptr, y, N, residual, rows, N, K, wfmt, act, epi, 1};
+        e = launch_rmsnorm(ctx->stream, x, K, norm_w, ctx->scratch, K, rows, K, eps, act);
+        GemmArgs m{ctx->scratch, K, w, nullptr, y, N, residual, rows, N, K, wfmt, act, epi, 1};
         if (e == hipSuccess) e = launch_gemm(ctx->stream, m);
     } else {
-        e = pack_rows_ok(ctx, g) ? pack_rows(ctx, g) : hipSuccess;
+        e = pack_rows_ok(g) ? pack_rows(ctx, g) : hipSuccess;
         if (e == hipSuccess) e = launch_gemv(ctx->stream, g);
     }
     lk.unlock();
@@ -369,7 +365,7 @@ int lssm_inproj_decode(lssm_ctx* ctx, const void* hidden, const void* norm_w, co
     hipError_t e = hipSuccess;
     {
         std::lock_guard<std::mutex> lk(ctx->scratch_mu);
-        if (pack_rows_ok(ctx, a.g)) e = pack_rows(ctx, a.g);
+        if (pack_rows_ok(a.g)) e = pack_rows(ctx, a.g);
         if (e == hipSuccess) e = launch_inproj_decode(ctx->stream, a);
     }
     if (e != hipSuccess) return set_error(LSSM_EDEVICE, "inproj_decode: %s", hipGetErrorString(e));

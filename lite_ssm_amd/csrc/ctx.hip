@@ -108,7 +108,7 @@ int lssm_ctx_create(lssm_ctx** out, void* stream) {
         c->own_stream = true;
     }
     e = hipMalloc((void**)&c->status, 256);
-    if (e == hipSuccess) e = hipMalloc(&c->xpack, GEMV_PACK_BYTES);
+    if (e == hipSuccess) e = hipMalloc(&c->scratch, CTX_SCRATCH_BYTES);
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->status_host, 256, hipHostMallocDefault);
     if (e == hipSuccess) {
         *c->status_host = 0;
@@ -117,7 +117,7 @@ int lssm_ctx_create(lssm_ctx** out, void* stream) {
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         if (c->status) (void)hipFree(c->status);
-        if (c->xpack) (void)hipFree(c->xpack);
+        if (c->scratch) (void)hipFree(c->scratch);
         if (c->status_host) (void)hipHostFree(c->status_host);
         if (c->own_stream) (void)hipStreamDestroy(c->stream);
         delete c;
@@ -133,9 +133,8 @@ int lssm_ctx_destroy(lssm_ctx* ctx) {
     // An uncommitted batch is dropped after the queued work drains (ops.mm:64-68).
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipFree(ctx->status);
-    (void)hipFree(ctx->xpack);
+    (void)hipFree(ctx->scratch);
     (void)hipHostFree(ctx->status_host);
-    if (ctx->gemm_ws) (void)hipFree(ctx->gemm_ws);
     if (ctx->ssd_seg) (void)hipFree(ctx->ssd_seg);
     if (ctx->ssd_gram) (void)hipFree(ctx->ssd_gram);
     for (float* p : ctx->ssd_gram_retired) (void)hipFree(p);

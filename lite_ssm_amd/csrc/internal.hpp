@@ -37,15 +37,13 @@ struct lssm_ctx {
     float* ssd_gram = nullptr;
     size_t ssd_gram_cap = 0;   // floats
     std::vector<float*> ssd_gram_retired;
-    // split-K slices of lssm_linear's GEMM (lssm::GEMM_WS_FLOATS), allocated by
-    // the first call that splits outside a stream capture
-    float* gemm_ws = nullptr;
-    // x rows packed for the batched decode GEMV (lssm::GEMV_PACK_BYTES)
-    void* xpack = nullptr;
-    // held while a call enqueues the launches that pass gemm_ws or xpack on to
-    // each other (two threads on one context).  A call that is captured uses
-    // neither: its graph may be replayed beside the context's other work, on
-    // other streams and after the context.
+    // What a call's launches pass on to each other, allocated with the context:
+    // split-K slices of lssm_linear's GEMM (lssm::GEMM_WS_FLOATS) or x rows
+    // packed for the batched decode GEMV (lssm::GEMV_PACK_BYTES)
+    void* scratch = nullptr;
+    // held while a call enqueues such launches (two threads on one context).  A
+    // call that is captured does not use the scratch: its graph may be replayed
+    // beside the context's other work, on other streams and after the context.
     std::mutex scratch_mu;
 };
 
@@ -464,6 +462,8 @@ bool launch_gemv_rows(hipStream_t s, const GemvArgs& a, hipError_t& err);
 bool launch_inproj_rows(hipStream_t s, const InprojDecodeArgs& a, hipError_t& err);
 // Bytes of x packed for it, at most.
 constexpr size_t GEMV_PACK_BYTES = (size_t)64 * 8192 * 2;
+constexpr size_t CTX_SCRATCH_BYTES = GEMM_WS_FLOATS * sizeof(float);
+static_assert(CTX_SCRATCH_BYTES >= GEMV_PACK_BYTES, "one buffer holds either");
 // Partials per row (N / 16) the single-pass MFMA GEMV writes for (M, N, K)
 // with GemvArgs::yfrag, or 0 when it cannot (another plan, or a count the
 // GEMV that reads them does not take).

@@ -1,6 +1,7 @@
 """Linear entries enqueued while a stream is captured: the graphs hold the
 caller's buffers only, so they are replayed side by side on two streams, beside
-eager calls of the same context and after it is destroyed."""
+eager calls of the same context and after it is destroyed; and eager calls
+while another stream is captured."""
 import numpy as np
 import pytest
 import torch
@@ -160,3 +161,32 @@ def test_captured_linears_hold_no_context_memory(ctx, rng, kind):
     c2.close()
     for k, g, ref in zip(calls, graphs, want):
         assert all(torch.equal(a, b) for a, b in zip(_solo(k, g.replay), ref))
+
+
+def test_first_split_call_allocates_nothing(ctx, rng):
+    """A context's first lssm_linear that splits K allocates no memory, which a
+    capture of another stream (global mode) would refuse and be ended by."""
+    import lite_ssm_amd as L
+    print("case: first split linear of a context beside a capture", flush=True)
+    k = _Linear(rng, *_Linear.weights(rng))
+    want = _solo(k, lambda: k.call(ctx))                 # (code loaded)
+    st, cap = torch.cuda.Stream(), torch.cuda.Stream()
+    c2 = L.Ctx(st.cuda_stream)
+    a = torch.zeros(1000, device="cuda")
+    k.reset()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    c2.begin_batch()
+    with torch.cuda.stream(cap):
+        g.capture_begin(capture_error_mode="global")
+        a.add_(1)
+        k.call(c2)
+        g.capture_end()
+    c2.commit_and_wait()
+    assert torch.equal(k.y, want[0])
+    assert free - torch.cuda.mem_get_info()[0] < 16 << 20
+    g.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(a, torch.ones_like(a))
+    c2.close()
