@@ -578,7 +578,7 @@ __global__ __launch_bounds__(64 * (CW + 4)) void gemm2_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Skinny GEMM for few rows (up to 48): the weights are streamed once.
+// Skinny GEMM for few rows (up to 64): the weights are streamed once.
 // A block covers 16 rows of W; its KS waves split K into slices of UPW units,
 // and the slices are summed in LDS.  A lane loads 16 bytes of one W row per
 // unit (int4: 32 k, int8: 16, dense: 8) and dequantizes them (to r(q s), GEMM
@@ -779,8 +779,9 @@ template <int FMT> int skinny_upw(uint32_t K, int mt) {
 
 template <int FMT, typename T, int MT>
 hipError_t go_skinny_mt(hipStream_t s, const GemmArgs& a, int upw) {
-    // (quantized weights past 16 rows, K <= 2048: one or two units always do)
-    if constexpr (MT == 1 || FMT == LSSM_W_DENSE)
+    // (quantized weights past 16 rows, K <= 2048, and any past 48, K <= 1024:
+    // one or two units always do)
+    if constexpr (MT == 1 || (FMT == LSSM_W_DENSE && MT < 4))
         if (upw == 4) return go_skinny<FMT, T, MT, 4>(s, a);
     if (upw == 2) return go_skinny<FMT, T, MT, 2>(s, a);
     return go_skinny<FMT, T, MT, 1>(s, a);
@@ -826,9 +827,11 @@ inline bool gemm_takes_mid(const GemmArgs& a) {
 // Units per wave of the skinny kernel for a call, 0 where it does not take it:
 // few rows, weights streamed once.  Every block reads all of x, so past 16 rows
 // only while that is small (us, here / gemm_mid): 37 x 10576 x 2560 int4 26.2 /
-// 15.2, 32 x 768 x 1536 int8 7.0 / 9.2, 37 x 3352 x 768 int8 6.2 / 7.5.
+// 15.2, 32 x 768 x 1536 int8 7.0 / 9.2, 37 x 3352 x 768 int8 6.2 / 7.5.  Past 48
+// rows K 768 only is the faster one throughout (49 rows 5.1 / 6.9, 64 rows 5.7 /
+// 6.9 int8, 5.9 / 6.0 dense; at K 1536 7.6 / 8.6 int4, 9.4 / 8.6 dense).
 template <int FMT> int skinny_takes(const GemmArgs& a) {
-    if (a.M > 48 || (a.M > 16 && a.K > 2048)) return 0;
+    if (a.M > 64 || (a.M > 48 && a.K > 1024) || (a.M > 16 && a.K > 2048)) return 0;
     return skinny_upw<FMT>(a.K, (int)(a.M + 15) / 16);
 }
 
@@ -837,7 +840,8 @@ hipError_t go_epi(hipStream_t s, const GemmArgs& a) {
     if (const int upw = skinny_takes<FMT>(a)) {
         if (a.M <= 16) return go_skinny_mt<FMT, T, 1>(s, a, upw);
         if (a.M <= 32) return go_skinny_mt<FMT, T, 2>(s, a, upw);
-        return go_skinny_mt<FMT, T, 3>(s, a, upw);
+        if (a.M <= 48) return go_skinny_mt<FMT, T, 3>(s, a, upw);
+        return go_skinny_mt<FMT, T, 4>(s, a, upw);
     }
     if (gemm_takes_mid(a)) return launch_gemm_mid(s, a, gemm_mid_plan(a));
     // the large tile for prefill-sized M; X byte offsets within a 256-row
