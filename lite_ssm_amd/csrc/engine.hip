@@ -294,8 +294,17 @@ struct lssm_engine {
         // packed for the single-pass kernel, or for gemv_rows
         const bool frag_in = B >= PACK_MIN_ROWS && mmx_in && gemv_mma_takes(B, proj, d_model, wfmt, act);
         const bool frag_out = B >= PACK_MIN_ROWS && mmx_out && gemv_mma_takes(B, d_model, d_inner, wfmt, act);
-        const bool rows_in = !frag_in && rows_aligned && gemv_rows_pays(B, proj, d_model, wfmt, act);
-        const bool rows_out = !frag_out && rows_aligned && gemv_rows_pays(B, d_model, d_inner, wfmt, act);
+        // (int4 x fp16 already from 15 rows: in a graph the pack launch costs
+        // less than in a stream of calls.  130M, four steps of 16 rows: 2240 ->
+        // 2171 (32-groups) and 2232 -> 2151 us (64-groups); 14 rows and bf16 the
+        // same either way, int8 and dense slower)
+        const bool q4_f16 = act == LSSM_F16 && (wfmt == LSSM_W_Q4_B32 || wfmt == LSSM_W_Q4_G64);
+        auto rows_pay = [&](uint32_t n, uint32_t k) {
+            return rows_aligned && (gemv_rows_pays(B, n, k, wfmt, act) ||
+                                    (q4_f16 && B >= 15 && gemv_rows_takes(B, n, k, wfmt, act)));
+        };
+        const bool rows_in = !frag_in && rows_pay(proj, d_model);
+        const bool rows_out = !frag_out && rows_pay(d_model, d_inner);
         const bool pack_in = frag_in || rows_in, pack_out = frag_out || rows_out;
         // fused RMSNorm + linear kernels: the VALU GEMV up to 4 rows, the MFMA
         // GEMVs for decode batches of the shapes they take

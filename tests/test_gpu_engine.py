@@ -200,14 +200,14 @@ PACK_CASES = [("f16-q8g32", O.F16, O.W_Q8_G32), ("f16-q4b32", O.F16, O.W_Q4_B32)
               ("bf16-q4g64", O.BF16, O.W_Q4_G64), ("f16-dense", O.F16, O.W_DENSE)]
 
 
-@pytest.mark.parametrize("B", [8, 24, 32])
+@pytest.mark.parametrize("B", [8, 16, 24, 32])
 @pytest.mark.parametrize("tag,act,wfmt", PACK_CASES, ids=[c[0] for c in PACK_CASES])
 def test_engine_batch8_packed_staging(ctx, tag, act, wfmt, B):
-    """Decode batches from 8 rows take the packing pass (x normalised and
-    packed once per linear) and the single-pass MFMA GEMV, which reads the
-    packed rows straight from memory: 8 and 24/32 rows (one and two tiles of
-    16 batch rows), for every format the MFMA GEMV takes; against the
-    oracle's per-sequence decode."""
+    """Decode batches of 8 to 32 rows at the 130M widths (one and two tiles of
+    16 batch rows), against the oracle's per-sequence decode.  int4 group 64 x
+    bf16 packs x once per linear for the single-pass MFMA GEMV; the other
+    formats normalise it in the staging MFMA GEMV's blocks at 8 rows, and pack it
+    for the batched GEMV at 16 rows (int4 x fp16) and past them."""
     from lite_ssm_amd.model import Engine
     print(f"case: packed decode {tag} batch {B}", flush=True)
     L, sh, m, om = _setup(ctx, "mamba2-130m", act, wfmt, n_layer=2, vocab_size=1024, seed=17)
