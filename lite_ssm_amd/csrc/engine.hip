@@ -258,8 +258,10 @@ struct lssm_engine {
                 if (e != hipErrorNotSupported) return e;
             }
             e = launch_gemv(st(), g);
-        } else if (rows_aligned && gemv_rows_pays(rows, vocab, d_model, LSSM_W_DENSE, act)) {
-            // norm_f into the packed rows, W streamed once
+        } else if (rows >= 12 && rows_aligned && gemv_rows_pays(rows, vocab, d_model, LSSM_W_DENSE, act)) {
+            // norm_f into the packed rows, W streamed once (fewer rows: norm and
+            // GEMM of few rows, 50280 x 768: 20.0 against 21.7 us at 6 rows, 23.5
+            // against 23.3 at 14)
             e = launch_mma_pack(st(), x, xs, norm_f, RMS_EPS, rows, d_model, LSSM_W_DENSE, act, d_gn);
             GemvArgs g{x, xs, lm_head, nullptr, logits, vocab, nullptr, norm_f, RMS_EPS, rows, vocab,
                        d_model, LSSM_W_DENSE, act, LSSM_EPI_NONE};
