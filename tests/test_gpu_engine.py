@@ -197,7 +197,8 @@ def test_engine_batch8_decode(ctx):
 
 
 PACK_CASES = [("f16-q8g32", O.F16, O.W_Q8_G32), ("f16-q4b32", O.F16, O.W_Q4_B32),
-              ("bf16-q4g64", O.BF16, O.W_Q4_G64), ("f16-dense", O.F16, O.W_DENSE)]
+              ("bf16-q4g64", O.BF16, O.W_Q4_G64), ("f16-dense", O.F16, O.W_DENSE),
+              ("bf16-q8g32", O.BF16, O.W_Q8_G32)]
 
 
 @pytest.mark.parametrize("B", [8, 16, 24, 32])
@@ -205,8 +206,8 @@ PACK_CASES = [("f16-q8g32", O.F16, O.W_Q8_G32), ("f16-q4b32", O.F16, O.W_Q4_B32)
 def test_engine_batch8_packed_staging(ctx, tag, act, wfmt, B):
     """Decode batches of 8 to 32 rows at the 130M widths (one and two tiles of
     16 batch rows), against the oracle's per-sequence decode.  int4 group 64 x
-    bf16 packs x once per linear for the single-pass MFMA GEMV; the other
-    formats normalise it in the staging MFMA GEMV's blocks at 8 rows, and pack it
+    bf16 packs x once per linear for the single-pass MFMA GEMV, int8 x bf16 for
+    the batched one; the other formats normalise it in the staging MFMA GEMV's blocks at 8 rows, and pack it
     for the batched GEMV at 16 rows (int4 x fp16) and past them."""
     from lite_ssm_amd.model import Engine
     print(f"case: packed decode {tag} batch {B}", flush=True)
@@ -223,6 +224,46 @@ def test_engine_batch8_packed_staging(ctx, tag, act, wfmt, B):
             eng.decode(torch.from_numpy(tok).cuda(), nxt)
             ref = om.decode(conv, ssd, tok)
             _check_logits(eng.logits(B).float().cpu().numpy(), ref, act, f"{tag} b{B} decode {step}")
+            tok = O.argmax(ref, act)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("act,wfmt,B", [(O.F16, O.W_Q8_G32, 24), (O.F16, O.W_Q4_B32, 16), (O.BF16, O.W_Q4_G64, 8),
+                                        (O.BF16, O.W_Q8_G32, 12)])
+def test_engine_unaligned_weights_decode(ctx, act, wfmt, B):
+    """Norm weights and scales that start two bytes past an aligned address (a
+    file's tensors need not be aligned): the decode batches that would pack x
+    take the launches that do not need it."""
+    from lite_ssm_amd.model import Engine
+    print(f"case: unaligned weights act {act} fmt {wfmt} batch {B}", flush=True)
+    L, sh, m, om = _setup(ctx, "mamba2-130m", act, wfmt, n_layer=2, vocab_size=512, seed=29)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        view = buf[1:].view(t.shape)
+        view.copy_(t)
+        assert view.data_ptr() % 4 == 2
+        return view
+
+    for w in m.layers:
+        for name in ("norm_w", "mixer_norm_w", "in_proj_s", "out_proj_s"):
+            w[name] = shifted(w[name])
+    m.norm_f = shifted(m.norm_f)
+    torch.cuda.synchronize()
+    eng = Engine(ctx, m, max_batch=B, max_seq=20)
+    try:
+        ids = np.random.default_rng(6).integers(0, sh.vocab_size, (B, 20)).astype(np.int32)
+        nxt = torch.zeros(B, dtype=torch.int32, device="cuda")
+        eng.prefill(torch.from_numpy(ids).cuda(), nxt)
+        conv, ssd = om.new_state(B)
+        ref = om.prefill(conv, ssd, ids)
+        _check_logits(eng.logits(B).float().cpu().numpy(), ref, act, f"unaligned b{B} prefill")
+        tok = O.argmax(ref, act)
+        for step in range(2):
+            eng.decode(torch.from_numpy(tok).cuda(), nxt)
+            ref = om.decode(conv, ssd, tok)
+            _check_logits(eng.logits(B).float().cpu().numpy(), ref, act, f"unaligned b{B} decode {step}")
             tok = O.argmax(ref, act)
     finally:
         eng.close()
@@ -317,21 +358,20 @@ def test_engine_prefill_folded_norms(ctx, monkeypatch):
     epilogue writes the next layer's r(h w) with sums of h^2 per 128 columns
     and the next in_proj scales its fp32 sums by 1 / rms; the chunked scan's Y
     stores hold the gated norm's r(g w) with sums of g^2 and out_proj scales
-    by that 1 / rms.  Full-width 2.7B layers at 1600 rows (7 row tiles: the
-    out_proj GEMM runs unsplit, so the fold is taken): every layer against the
-    oracle's run_block on the engine's own input rows, and against an engine
-    with both folds off (LSSM_FOLD_PRE_NORM=0, LSSM_FUSED_GATED_NORM=0), which
-    must differ (the folds ran) but stay within the bound."""
+    by that 1 / rms.  Full-width 2.7B layers at 1700 rows (the large tiles by a
+    wide margin, which have the fold): every layer against the oracle's run_block
+    on the engine's own input rows, and against an engine with both folds off,
+    within the bound.  An engine with the gated norm's fold alone must differ
+    from both: each fold ran."""
     from lite_ssm_amd.model import Engine
-    print("case: folded prefill norms, 2.7B widths, 3 layers, 1 x 1600", flush=True)
+    print("case: folded prefill norms, 2.7B widths, 3 layers, 1 x 1700", flush=True)
     L, sh, m, om = _setup(ctx, "mamba2-2.7b", O.BF16, O.W_Q4_G64, n_layer=3, vocab_size=512, seed=37)
-    B, Lq = 1, 1600
+    B, Lq = 1, 1700
     ids = np.random.default_rng(9).integers(0, sh.vocab_size, (B, Lq)).astype(np.int32)
     traces = {}
-    for mode in ("off", "on"):
-        v = "0" if mode == "off" else "1"
-        monkeypatch.setenv("LSSM_FOLD_PRE_NORM", v)
-        monkeypatch.setenv("LSSM_FUSED_GATED_NORM", v)
+    for mode in ("off", "gated", "on"):
+        monkeypatch.setenv("LSSM_FOLD_PRE_NORM", "1" if mode == "on" else "0")
+        monkeypatch.setenv("LSSM_FUSED_GATED_NORM", "0" if mode == "off" else "1")
         eng = Engine(ctx, m, max_batch=B, max_seq=Lq)
         try:
             tr = torch.zeros((sh.n_layer + 1, B * Lq, sh.d_model), dtype=torch.bfloat16, device="cuda")
@@ -342,11 +382,11 @@ def test_engine_prefill_folded_norms(ctx, monkeypatch):
             traces[mode] = tr.view(torch.int16).cpu().numpy()
         finally:
             eng.close()
-    on, off = traces["on"], traces["off"]
+    on, off, gated = traces["on"], traces["off"], traces["gated"]
     assert np.array_equal(on[0], off[0]), "the embedding rows differ"
     conv, ssd = om.new_state(B)
     for li in range(sh.n_layer):
-        h = np.ascontiguousarray(on[li])
+        h = on[li].copy()                  # (the oracle works in place)
         om.block(li, h, conv, ssd, B, Lq, False)
         e = max_rel(O.from_act(h, O.BF16), O.from_act(on[li + 1], O.BF16))
         d = max_rel(O.from_act(on[li + 1], O.BF16), O.from_act(off[li + 1], O.BF16))
@@ -355,7 +395,9 @@ def test_engine_prefill_folded_norms(ctx, monkeypatch):
               f"({same:.3f} of elements equal)", flush=True)
         assert e <= MAXREL[O.BF16], f"layer {li}: output max-rel {e:.3e} against the oracle"
         assert d <= MAXREL[O.BF16], f"layer {li}: folded and unfolded differ by {d:.3e}"
-    assert not np.array_equal(on[2], off[2]), "the second layer's rows are bit-identical: no fold ran"
+    assert not np.array_equal(gated[1], off[1]), "the first layer's rows are bit-identical: the gated norm was not folded"
+    assert np.array_equal(on[1], gated[1]), "the first layer has no norm folded into its in_proj"
+    assert not np.array_equal(on[2], gated[2]), "the second layer's rows are bit-identical: the pre-norm was not folded"
 
 
 @pytest.mark.parametrize("name,act,wfmt,vocab", [
