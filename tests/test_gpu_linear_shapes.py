@@ -173,3 +173,84 @@ def test_small_tile_gemm_strides_epilogues(ctx, rng, act, M, N, K):
                 got = act_host(y, act)
                 assert_close(np.ascontiguousarray(got[:, :N]), ref, act, {O.F16: 2e-3, O.BF16: 1.6e-2}[act], "epilogue")
                 assert np.array_equal(got[:, N:], res[:, N:])
+
+
+# --------------------------------------------------------------------------- infinities, threads
+# One shape for each kernel: fp32 with a K step wider than K, few rows, small
+# tiles in one pass and split, and the batched decode GEMV.
+@pytest.mark.parametrize("act,wfmt,M,N,K", [(O.F32, O.W_Q8_G32, 40, 96, 96), (O.F32, O.W_DENSE, 40, 96, 96),
+                                            (O.F16, O.W_Q8_G32, 40, 70, 768), (O.BF16, O.W_DENSE, 100, 300, 320),
+                                            (O.F16, O.W_Q4_B32, 100, 300, 320), (O.BF16, O.W_Q4_G64, 70, 256, 5120)])
+def test_gemm_rows_with_infinities_leave_the_others(ctx, rng, act, wfmt, M, N, K):
+    """A row with an infinity or a NaN (at both ends of K) is non-finite; the
+    other rows keep their bits."""
+    print(f"case: infinities act {act} fmt {wfmt} {M} x {N} x {K}", flush=True)
+    x = rng.standard_normal((M, K))
+    w, s = _weights(rng, N, K, wfmt, act)
+    wd, sd = dev(w), _sdev(s)
+    out = []
+    for bad in (False, True):
+        if bad:
+            x[5, 0], x[17, K - 1], x[M - 1, 0] = np.inf, -np.inf, np.nan
+        y = empty((M, N), act)
+        ctx.linear(dev(O.to_act(x, act)), wd, sd, y, M, N, K, wfmt, act)
+        out.append(act_host(y, act))
+    hit = np.array([5, 17, M - 1])
+    assert not np.isfinite(O.from_act(out[1][hit], act)).any()
+    assert np.array_equal(np.delete(out[0], hit, 0), np.delete(out[1], hit, 0))
+
+
+@pytest.mark.parametrize("act,wfmt,M", [(O.BF16, O.W_Q8_G32, 24), (O.F16, O.W_Q4_B32, 33), (O.BF16, O.W_DENSE, 64)])
+def test_decode_rows_with_infinities_leave_the_others(ctx, rng, act, wfmt, M):
+    N, K = 300, 1280
+    print(f"case: infinities in decode rows act {act} fmt {wfmt} {M} x {N} x {K}", flush=True)
+    x = rng.standard_normal((M, K))
+    nw = O.to_act(1 + 0.1 * rng.standard_normal(K), act)
+    w, s = _weights(rng, N, K, wfmt, act)
+    clean = _norm_linear(ctx, O.to_act(x, act), nw, w, s, M, N, K, wfmt, act)
+    x[3, 0], x[18, K - 1], x[M - 1, 640] = np.inf, -np.inf, np.nan
+    got = _norm_linear(ctx, O.to_act(x, act), nw, w, s, M, N, K, wfmt, act)
+    hit = np.array([3, 18, M - 1])
+    assert not np.isfinite(O.from_act(got[hit], act)).any()
+    assert np.array_equal(np.delete(clean, hit, 0), np.delete(got, hit, 0))
+
+
+def test_two_threads_share_a_context(ctx, rng):
+    """Calls that pass data on in the context's scratch, from two threads: packed
+    rows in one, split K in the other."""
+    import threading
+    import lite_ssm_amd as L
+    print("case: two threads on one context", flush=True)
+    M, N, K, act = 24, 300, 2560, O.BF16
+    nw = dev(O.to_act(1 + 0.1 * rng.standard_normal(K), act))
+    w, s = (dev(a) for a in _weights(rng, N, K, O.W_Q8_G32, act))
+    x, y = dev(O.to_act(rng.standard_normal((M, K)), act)), empty((M, N), act)
+    M2, N2, K2 = 70, 256, 5120
+    w2, s2 = (dev(a) for a in _weights(rng, N2, K2, O.W_Q4_G64, act))
+    x2, y2 = dev(O.to_act(rng.standard_normal((M2, K2)), act)), empty((M2, N2), act)
+
+    def rows():
+        L.check(L.lib.lssm_norm_linear_decode(ctx.h, x.data_ptr(), nw.data_ptr(), 1e-5, w.data_ptr(), s.data_ptr(),
+                                              y.data_ptr(), None, M, N, K, O.W_Q8_G32, act, L.EPI_NONE))
+
+    def split():
+        ctx.linear(x2, w2, s2, y2, M2, N2, K2, O.W_Q4_G64, act)
+
+    rows()
+    split()
+    want = act_host(y, act).copy(), act_host(y2, act).copy()
+    wrong = []
+
+    def loop(call, out, ref):
+        # (numpy copies of the outputs: the calls themselves return when done)
+        for _ in range(50):
+            call()
+        if not np.array_equal(act_host(out, act), ref):
+            wrong.append(call.__name__)
+
+    both = [threading.Thread(target=loop, args=a) for a in ((rows, y, want[0]), (split, y2, want[1]))]
+    for t in both:
+        t.start()
+    for t in both:
+        t.join(30)
+    assert not wrong and not any(t.is_alive() for t in both)

@@ -503,6 +503,8 @@ INPROJ_CASES = [
     (O.F16, O.W_Q4_B32, 33, 2560), (O.F16, O.W_Q8_G32, 16, 2560), (O.F16, O.W_DENSE, 7, 2560),
     # K = 5120: 16 rows take two passes of 8 (staging does not fit 16)
     (O.BF16, O.W_Q4_G64, 16, 5120), (O.F16, O.W_Q8_G32, 12, 5120),
+    # formats of the batched GEMV over packed rows only
+    (O.BF16, O.W_Q8_G32, 24, 4096), (O.BF16, O.W_Q8_G32, 33, 2560), (O.BF16, O.W_DENSE, 17, 2560),
     # 8B in_proj shape at batch 32 (4 tiles per block, 2 passes)
     (O.BF16, O.W_Q4_G64, 32, 4096),
 ]
