@@ -225,7 +225,7 @@ bool gemm_norm_fold_takes(const GemmArgs& a);
 hipError_t launch_gemm(hipStream_t s, const GemmArgs& a);
 // Workspace the engine and the contexts give launch_gemm for its split-K
 // slices (floats).
-constexpr size_t GEMM_WS_FLOATS = (size_t)8 << 20;   // 32 MiB
+constexpr size_t GEMM_WS_FLOATS = (size_t)4 << 20;   // 16 MiB: a 128 x 128 tile of sums for each of 256 CUs, the most a plan takes
 // The same product in smaller tiles (gemm_mid.hip) for grids that leave CUs
 // idle: bm x bn tiles, K in `split` slices (more than one only with a.ws) and
 // an estimate of its time; cost ~0 and bm 0 where it does not take the call.
