@@ -10,8 +10,11 @@
 // and split every K step (their sums meet in LDS), so that a grid of few tiles
 // can be cut finer:
 //   64 x 64 (four waves, KW 1), 32 x 64 (four, KW 2), 32 x 32 (eight, KW 8)
-// A K step is 32 KW wide.  Loads run two steps ahead in two register sets,
-// LDS is double-buffered, one barrier per step.  LDS rows are padded by 16
+// A K step is 32 KW wide.  Two register sets, loads two steps ahead as written:
+// as compiled the tiles of 32 rows request a step's loads near the end of the
+// step before it is stored and wait for them among the next MFMAs (300 x 3352 x
+// 768, 26 us: MFMA 49 % busy; the waves wait to issue two thirds of their cycles).  LDS
+// is double-buffered, one barrier per step.  LDS rows are padded by 16
 // bytes (pitch 4 mod 64 banks): the 16-byte fragment reads of 16 consecutive
 // rows hit distinct banks.  A lane reads four consecutive k of its row for
 // four MFMAs: the k order inside the product is the same for both operands.

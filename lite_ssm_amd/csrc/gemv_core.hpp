@@ -28,8 +28,8 @@ struct GemvCore {
     float eps;
     uint32_t N, K;
     float inv_k;                                     // 1 / K (the RMSNorm mean)
-    // the MFMA decode GEMV only: x already normalised and packed in its
-    // staging order ([M][K / 2] dwords, launch_mma_pack), or null
+    // the MFMA decode GEMVs only: x already normalised and packed in fragment
+    // order (launch_mma_pack), or null
     const uint32_t* xp = nullptr;
     // gemv_mmx only, with xp: when part is set, xp holds the rows raw (not
     // normalised) in fragment order, their sums of squares are the `nparts`

@@ -898,7 +898,7 @@ __global__ __launch_bounds__(64 * MMX_MAXW) void gemv_mmx_kernel(GemvCore c, Epi
     if constexpr (epi_tail<Epi>::value) epi.tail();
 }
 
-// LSSM_MMA_STAGED=1 (read once) keeps packed x on the staging kernel, for A/B
+// LSSM_MMA_STAGED=1 (read once) turns the single-pass kernel off, for A/B
 // measurements.
 inline bool mmx_disabled() {
     static const bool off = [] {

@@ -18,8 +18,9 @@ namespace {
 // W rows and all RT tiles of 16 batch rows, so W is read from memory once
 // whatever the batch; x is re-read by every block from L2 (RT KB per 32 k,
 // against CT tiles of W), which CT keeps near the W traffic.
-// Bound by the W stream, by the unpack's VALU work for int8 x bf16 and 33 rows
-// and more of int4.
+// Bound by latency: 18560 x 4096 int8 x bf16 at 24 rows streams its 81 MB in 26.6
+// us (3.1 TB/s) in one round of blocks of four ring turns each; VALU issue takes
+// 28 % of the cycles, the MFMA pipe 8 %.
 // (A ring of four: slower at every shape, its registers cost more than the
 // loads in flight bring.  A persistent grid of such blocks over many tiles:
 // the waves meet after every group, and the loop-carried ring spilled.)
@@ -112,7 +113,8 @@ __global__ __launch_bounds__(64 * GR_W) void gemv_rows_kernel(GemvCore c, Epi ep
         wp[t] = c.w + n * F::row_bytes(K) + 16 * lq;
         sp[t] = P::G > 0 ? reinterpret_cast<const uint32_t*>(c.s + n * (K / (P::G > 0 ? P::G : 1))) : nullptr;
     }
-    // quads past the wave's last re-read it (their products are skipped)
+    // past the wave's last quad the next wave's are read, past the row's end its
+    // last again (their products are skipped)
     auto load = [&](uint32_t q, Slot& r) {
         const uint32_t qa = min(q, quads - 1);
 #pragma unroll

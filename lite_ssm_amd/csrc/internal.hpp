@@ -151,7 +151,7 @@ struct GemvArgs {
     uint32_t M, N, K;
     int wfmt, act, epi;
     // x rows as launch_mma_pack wrote them (norm_w applied), or null; used by
-    // the MFMA decode GEMV, which then copies instead of normalising
+    // the MFMA decode GEMVs, which then read instead of normalising
     const void* xpack = nullptr;
     // the gemv_rows kernel takes the call (gemv_rows_takes): x from xpack, or
     // where that is null normalised by every block (norm_w; 16-byte aligned)
@@ -447,8 +447,8 @@ bool gemv_rows_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
 // Dense weights of so many rows (the lm_head) that the tiled GEMM behind a norm
 // launch streams them faster, past four rows of x: it reads them in runs of
 // 128 bytes a row, a tile's rows at a time (50280 x 2560 at 16 rows: 57.6
-// against 68 us; at K below 2048 gemv_rows is ahead: 50280 x 768 15 against
-// 20.9).
+// against 68 us; at K below 2048 gemv_rows is ahead: 50280 x 768 at 16 rows 18.8
+// against 20.8).
 bool dense_head_gemm(uint32_t N, uint32_t K, int wfmt, int act);
 // Whether packing x and running it is the fastest way to take a decode linear
 // of M rows with its RMSNorm.
