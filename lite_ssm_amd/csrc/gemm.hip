@@ -605,7 +605,11 @@ template <typename T> __device__ __forceinline__ floatx4 mma16x32(u32x4 a, u32x4
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
 }
 
-template <int FMT, typename T, int EPI, int MT, int UPW>
+// TWO: within 64 registers, so that a CU holds two blocks of 15 or 16 waves
+// (28 waves fit otherwise): wave 0 keeps its sum, the residual and the row scale
+// come behind the sums.  For int8 and one row tile, which it fits (18560 x 4096
+// at 13 rows: 34.2 us, with one block a CU 37.0).
+template <int FMT, typename T, int EPI, int MT, int UPW, bool TWO = false>
 __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
     using SU = SkUnit<FMT>;
     constexpr int KPL = SU::KPL, U = SU::U, STEPS = SU::STEPS;
@@ -617,7 +621,7 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
     const int li = lane % 16, lq = lane / 16;
     const uint32_t n0 = blockIdx.x * 16;
     const uint32_t K = a.K, KS = K / (UPW * U);
-    const uint32_t kb = min((uint32_t)w, KS - 1) * (UPW * U);   // (waves past KS only finish a tile)
+    const uint32_t kb = (TWO ? (uint32_t)w : min((uint32_t)w, KS - 1)) * (UPW * U);   // (waves past KS only finish a tile)
     const uint32_t n = min(n0 + li, a.N - 1);
 
     const char* wrow;
@@ -650,12 +654,13 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
     const bool own = w < MT && mo < a.M;
     T res[4];
     float rs = 1.0f;
-    if (own) {
+    auto load_out = [&] {
         if (a.row_scale) rs = a.row_scale[mo];
         if (EPI == LSSM_EPI_ADD)
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) res[rr] = ((const T*)a.res)[(size_t)mo * a.y_stride + min(no + rr, a.N - 1)];
-    }
+    };
+    if (!TWO && own) load_out();
     // all loads in flight before the first MFMA (when they fit the registers:
     // 16-wave blocks leave 128 VGPRs)
     if constexpr (UPW * MT <= 4) __builtin_amdgcn_sched_barrier(0);
@@ -692,14 +697,18 @@ __global__ __launch_bounds__(64 * SK_MAXW) void gemm_skinny_kernel(GemmArgs a) {
     // sum the K slices in order; waves 0 .. MT - 1 a row tile each (the launcher
     // gives the block MT waves).  D element r of lane l: row 4 (l / 16) + r (W row
     // n0 + .), column l % 16 (x row 16 mt + .).
-    if (w < (int)KS) {
+    if (TWO ? w > 0 : w < (int)KS) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) red[w][mt][lane] = acc[mt];
     }
     __syncthreads();
     if (!own) return;
+    if constexpr (TWO) {
+        load_out();
+        __builtin_amdgcn_s_waitcnt(0x0F70);              // vmcnt(0) here: else before each of the stores
+    }
     T* Y = (T*)a.y;
-    floatx4 v = red[0][w][lane];
+    floatx4 v = TWO ? acc[0] : red[0][w][lane];
     for (uint32_t q = 1; q < KS; ++q) v += red[q][w][lane];
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
@@ -753,14 +762,14 @@ __global__ void gemm_simple_kernel(GemmArgs a) {
     ((T*)a.y)[yi] = from_f<T>(v);
 }
 
-template <int FMT, typename T, int MT, int UPW>
+template <int FMT, typename T, int MT, int UPW, bool TWO = false>
 hipError_t go_skinny(hipStream_t s, const GemmArgs& a) {
     const dim3 grid((a.N + 15) / 16);
     const dim3 block(64 * std::max<uint32_t>(MT, a.K / (UPW * SkUnit<FMT>::U)));
     switch (a.epi) {
-        case LSSM_EPI_SILU: gemm_skinny_kernel<FMT, T, LSSM_EPI_SILU, MT, UPW><<<grid, block, 0, s>>>(a); break;
-        case LSSM_EPI_ADD: gemm_skinny_kernel<FMT, T, LSSM_EPI_ADD, MT, UPW><<<grid, block, 0, s>>>(a); break;
-        default: gemm_skinny_kernel<FMT, T, LSSM_EPI_NONE, MT, UPW><<<grid, block, 0, s>>>(a); break;
+        case LSSM_EPI_SILU: gemm_skinny_kernel<FMT, T, LSSM_EPI_SILU, MT, UPW, TWO><<<grid, block, 0, s>>>(a); break;
+        case LSSM_EPI_ADD: gemm_skinny_kernel<FMT, T, LSSM_EPI_ADD, MT, UPW, TWO><<<grid, block, 0, s>>>(a); break;
+        default: gemm_skinny_kernel<FMT, T, LSSM_EPI_NONE, MT, UPW, TWO><<<grid, block, 0, s>>>(a); break;
     }
     return hipGetLastError();
 }
@@ -779,12 +788,16 @@ template <int FMT> int skinny_upw(uint32_t K, int mt) {
 
 template <int FMT, typename T, int MT>
 hipError_t go_skinny_mt(hipStream_t s, const GemmArgs& a, int upw) {
-    // (quantized weights past 16 rows, K <= 2048, and any past 48, K <= 1024:
-    // one or two units always do)
-    if constexpr (MT == 1 || (FMT == LSSM_W_DENSE && MT < 4))
+    // (the units that skinny_upw gives: past 16 rows K <= 2048, past 48 K <= 1024)
+    constexpr bool DENSE = FMT == LSSM_W_DENSE, Q8 = FMT == LSSM_W_Q8_G32;
+    if constexpr (Q8 && MT == 1)
+        if (upw == 4 && a.K > 14 * 4 * SkUnit<FMT>::U) return go_skinny<FMT, T, MT, 4, true>(s, a);
+    if constexpr (MT == 1 || (DENSE && MT < 4))
         if (upw == 4) return go_skinny<FMT, T, MT, 4>(s, a);
-    if (upw == 2) return go_skinny<FMT, T, MT, 2>(s, a);
-    return go_skinny<FMT, T, MT, 1>(s, a);
+    if constexpr (MT <= 2 || DENSE || (Q8 && MT == 3))
+        if (upw == 2) return go_skinny<FMT, T, MT, 2>(s, a);
+    if (upw == 1) return go_skinny<FMT, T, MT, 1>(s, a);
+    return hipErrorInvalidValue;
 }
 
 // gemm2_kernel's tiles for a call.  256-wide tiles halve the X re-reads: a wide

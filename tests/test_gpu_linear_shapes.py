@@ -131,16 +131,16 @@ def test_gemv_int8_bf16(ctx, rng, M, K):
 # --------------------------------------------------------------------------- small-tile GEMM
 # Rows at the edges of the 64- and 128-row tiles, partial tiles in N, depths of
 # 1, 2, 3, 5 and 13 K steps, K deep enough to be split, and enough columns for
-# each of the three tiles; the largest has more tiles than CUs.  The last five:
-# the most rows of the kernel for few, with fewer K slices than row tiles too,
-# and at both ends of its 49 to 64 rows.
+# each of the three tiles; the largest has more tiles than CUs.  The last seven:
+# the most rows of the kernel for few, with fewer K slices than row tiles too, at
+# both ends of its 49 to 64 rows, and 15 and 16 slices of int8.
 @pytest.mark.parametrize("act", [O.F16, O.BF16])
 @pytest.mark.parametrize("wfmt", ALL_FMTS)
 @pytest.mark.parametrize("M,N,K", [(33, 200, 64), (63, 72, 1088), (64, 64, 128), (65, 130, 192), (127, 500, 320),
                                    (129, 1000, 832), (300, 1100, 2560), (17, 40, 5120), (12, 300, 8192),
                                    (100, 9000, 192), (300, 6000, 128), (700, 2560, 320), (1000, 2000, 128),
                                    (37, 200, 1536), (48, 40, 2048), (40, 40, 64),
-                                   (49, 200, 768), (64, 300, 1024)])
+                                   (49, 200, 768), (64, 300, 1024), (5, 40, 3840), (16, 200, 4096)])
 def test_small_tile_gemm_vs_oracle(ctx, rng, act, wfmt, M, N, K):
     print(f"case: small-tile GEMM act {act} fmt {wfmt} {M} x {N} x {K}", flush=True)
     x = O.to_act(rng.standard_normal((M, K)), act)
@@ -152,12 +152,13 @@ def test_small_tile_gemm_vs_oracle(ctx, rng, act, wfmt, M, N, K):
 
 
 @pytest.mark.parametrize("act", [O.F16, O.BF16])
-@pytest.mark.parametrize("M,N,K", [(37, 130, 192), (70, 256, 5120)])
+@pytest.mark.parametrize("M,N,K", [(37, 130, 192), (70, 256, 5120), (13, 130, 4096)])
 def test_small_tile_gemm_strides_epilogues(ctx, rng, act, M, N, K):
     """Padded rows (an odd y stride: element stores), SiLU and the in-place
-    residual, in one pass and (K = 5120) through the slices' sum."""
+    residual, in one pass, (K = 5120) through the slices' sum and (K = 4096) in
+    the kernel for few rows."""
     import lite_ssm_amd as L
-    for wfmt in (O.W_DENSE, O.W_Q4_G64):
+    for wfmt in (O.W_DENSE, O.W_Q4_G64, O.W_Q8_G32):
         w, s = _weights(rng, N, K, wfmt, act)
         xp = O.to_act(rng.standard_normal((M, K + 8)), act)
         x = np.ascontiguousarray(xp[:, :K])
