@@ -302,12 +302,21 @@ struct lssm_engine {
         // same either way, int8 and dense slower)
         const bool q4_f16 = act == LSSM_F16 && (wfmt == LSSM_W_Q4_B32 || wfmt == LSSM_W_Q4_G64);
         auto rows_pay = [&](uint32_t n, uint32_t k) {
+            const uint64_t staged = gemv_mma_staged(B, n, k, wfmt, act);
+            if (B < 8 && staged != 0 && staged <= 42000) return false;
             return rows_aligned && (gemv_rows_pays(B, n, k, wfmt, act) ||
                                     (q4_f16 && B >= 15 && gemv_rows_takes(B, n, k, wfmt, act)));
         };
-        const bool rows_in = !frag_in && rows_pay(proj, d_model);
-        const bool rows_out = !frag_out && rows_pay(d_model, d_inner);
-        const bool pack_in = frag_in || rows_in, pack_out = frag_out || rows_out;
+        // 5 to 7 rows are normalised in the staging kernel's blocks (to 42000
+        // values a CU; 2.7B, four layers and steps, 6 rows: int8 x fp16 935 with
+        // pack launches, 917 without, int4 786 and 761), 8 to 14 packed for it
+        // (8 rows 938 and 788, with gemv_rows 961 and 820; 16 rows 1123 and 976,
+        // with gemv_rows 1078 and 967)
+        const bool stg_in = !frag_in && rows_aligned && gemv_mma_packed_pays(B, proj, d_model, wfmt, act);
+        const bool stg_out = !frag_out && rows_aligned && gemv_mma_packed_pays(B, d_model, d_inner, wfmt, act);
+        const bool rows_in = !frag_in && !stg_in && rows_pay(proj, d_model);
+        const bool rows_out = !frag_out && !stg_out && rows_pay(d_model, d_inner);
+        const bool pack_in = frag_in || stg_in || rows_in, pack_out = frag_out || stg_out || rows_out;
         // fused RMSNorm + linear kernels: the VALU GEMV up to 4 rows, the MFMA
         // GEMVs for decode batches of the shapes they take
         const bool fused_in = (B <= 4 && (int)B <= gemv_max_rows(d_model, wfmt, act)) ||
@@ -370,7 +379,7 @@ struct lssm_engine {
                         // linear then rounds at the same point)
                         const bool raw = raw_pack || frag_parts;
                         e = launch_mma_pack(st(), d_hidden, d_model, w.norm_w, RMS_EPS, B, d_model, wfmt, act,
-                                            d_gn, raw ? h_part : nullptr);
+                                            d_gn, raw ? h_part : nullptr, stg_in);
                         a.g.xpack = d_gn;
                         a.g.xrows = rows_in;
                         if (raw) {
@@ -429,7 +438,7 @@ struct lssm_engine {
                     }
                 } else if (pack_out) {
                     e = launch_mma_pack(st(), d_g, d_inner, w.mixer_norm_w, RMS_EPS, B, d_inner, wfmt, act, d_gn,
-                                        raw_pack ? g_part : nullptr);
+                                        raw_pack ? g_part : nullptr, stg_out);
                     g.xpack = d_gn;
                     g.xrows = rows_out;
                     if (raw_pack) {

@@ -50,7 +50,8 @@ constexpr int MM_MAXJ = 8;                       // staged octets per thread and
 
 // ra: dwords of the LDS region that holds, in turn, the lanes' sums of
 // squares, the staged x rows and each pass's partial sums.
-template <int FMT, typename T, int CT, int QPW, bool NORM, class Epi>
+// PACKED: x (up to 16 rows, one pass) comes normalised from launch_mma_pack.
+template <int FMT, typename T, int CT, int QPW, bool NORM, bool PACKED, class Epi>
 __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvCore c, Epi epi, uint32_t M, uint32_t mpb,
                                                                  uint32_t ra) {
     using P = Mma<FMT, T>;
@@ -207,6 +208,26 @@ __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvC
         lds_barrier();
     };
 
+    // ---- packed x -> LDS: octet p = row * KO + cc, eight in flight per thread ----
+    auto copy_in = [&] {
+        const uint32_t NT = blockDim.x, n = M * KO;
+        const uint32_t ko_magic = 0xFFFFFFFFu / KO + 1u;           // KO >= 16: exact for p < 2^16
+        for (uint32_t p0 = threadIdx.x; p0 < n; p0 += 8 * NT) {
+            u32x4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t p = p0 + i * NT;
+                if (p < n) v[i] = reinterpret_cast<const u32x4*>(c.xp)[p];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t p = p0 + i * NT, r = __umulhi(p, ko_magic);
+                if (p < n) *reinterpret_cast<u32x4*>(xl + r * RS + 4 * (p - r * KO)) = v[i];
+            }
+        }
+        lds_barrier();
+    };
+
     // ---- weights (and raw scale bits) of the wave's quads, all in flight ----
     // With few weight registers (CT * QPW <= 8) they are held over all
     // passes; otherwise a later pass reads them again (L2 hits) rather than
@@ -250,7 +271,7 @@ __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvC
     // x of the first pass, staged before any weight is requested: requested
     // behind the weights, x would queue behind the whole chip's weight
     // traffic (measured: staging done ~7 us after the start instead of ~2)
-    const bool keep0 = mpb * SEG <= (uint32_t)(MM_MAXJ * KS);   // the first pass's x fits the registers
+    const bool keep0 = !PACKED && mpb * SEG <= (uint32_t)(MM_MAXJ * KS);   // the first pass's x fits the registers
     if (keep0) {
         const uint32_t nseg = mpb * SEG;
         const uint32_t lane0 = threadIdx.x % WAVE;
@@ -270,13 +291,14 @@ __global__ __launch_bounds__(64 * mma_waves(CT, QPW)) void gemv_mma_kernel(GemvC
             }
         }
     }
-    if (keep0) stage(0u, FmtTag<1>{});
+    if constexpr (PACKED) copy_in();
+    else if (keep0) stage(0u, FmtTag<1>{});
     else stage(0u, FmtTag<0>{});
     load_w();
 
     for (uint32_t base = 0; base < M; base += mpb) {
         if (base > 0) {
-            stage(base, FmtTag<0>{});
+            if constexpr (!PACKED) stage(base, FmtTag<0>{});
             if constexpr (!HOLD) load_w();
         }
         const uint32_t rows = min(mpb, M - base);
@@ -1071,9 +1093,9 @@ template <typename T> bool mma_aligned(const GemvCore& c, bool norm) {
            (!norm || (uintptr_t)c.norm_w % 16 == 0) && (uintptr_t)c.w % 16 == 0 && (uintptr_t)c.s % 16 == 0;
 }
 
-template <int FMT, typename T, int CT, int QPW, bool NORM, class Epi>
+template <int FMT, typename T, int CT, int QPW, bool NORM, bool PACKED, class Epi>
 hipError_t mma_run(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, const MmaPlan& p) {
-    auto k = gemv_mma_kernel<FMT, T, CT, QPW, NORM, Epi>;
+    auto k = gemv_mma_kernel<FMT, T, CT, QPW, NORM, PACKED, Epi>;
     // opt in to the dynamic LDS once per instantiation (a host attribute)
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MM_LDS_MAX);
@@ -1083,22 +1105,22 @@ hipError_t mma_run(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, c
     return hipGetLastError();
 }
 
-template <int FMT, typename T, bool NORM, class Epi>
+template <int FMT, typename T, bool NORM, bool PACKED, class Epi>
 hipError_t mma_shape(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, const MmaPlan& p) {
     if (p.ct == 1) {
         switch (p.qpw) {
-            case 1: return mma_run<FMT, T, 1, 1, NORM, Epi>(s, c, e, M, p);
-            case 2: return mma_run<FMT, T, 1, 2, NORM, Epi>(s, c, e, M, p);
-            case 4: return mma_run<FMT, T, 1, 4, NORM, Epi>(s, c, e, M, p);
-            default: return mma_run<FMT, T, 1, 8, NORM, Epi>(s, c, e, M, p);
+            case 1: return mma_run<FMT, T, 1, 1, NORM, PACKED, Epi>(s, c, e, M, p);
+            case 2: return mma_run<FMT, T, 1, 2, NORM, PACKED, Epi>(s, c, e, M, p);
+            case 4: return mma_run<FMT, T, 1, 4, NORM, PACKED, Epi>(s, c, e, M, p);
+            default: return mma_run<FMT, T, 1, 8, NORM, PACKED, Epi>(s, c, e, M, p);
         }
     }
     if constexpr (FMT == LSSM_W_Q4_G64 || FMT == LSSM_W_Q4_B32) {
-        if (p.qpw == 4) return mma_run<FMT, T, 4, 4, NORM, Epi>(s, c, e, M, p);
+        if (p.qpw == 4) return mma_run<FMT, T, 4, 4, NORM, PACKED, Epi>(s, c, e, M, p);
         switch (p.ct) {
-            case 2: return mma_run<FMT, T, 2, 2, NORM, Epi>(s, c, e, M, p);
-            case 3: return mma_run<FMT, T, 3, 2, NORM, Epi>(s, c, e, M, p);
-            default: return mma_run<FMT, T, 4, 2, NORM, Epi>(s, c, e, M, p);
+            case 2: return mma_run<FMT, T, 2, 2, NORM, PACKED, Epi>(s, c, e, M, p);
+            case 3: return mma_run<FMT, T, 3, 2, NORM, PACKED, Epi>(s, c, e, M, p);
+            default: return mma_run<FMT, T, 4, 2, NORM, PACKED, Epi>(s, c, e, M, p);
         }
     }
     return hipErrorInvalidValue;                       // not a planned shape
@@ -1152,11 +1174,12 @@ bool try_mma(hipStream_t s, const GemvCore& c, const Epi& e, uint32_t M, int wfm
             err = mmx_go<FMT, T, Epi>(s, c, e, M, q);
             return true;
         }
-        if (c.xp) {                                            // packed x: only the single-pass kernel
+        if (c.part || (c.xp && p.mpb < M)) {                   // raw x; more rows than one pass stages
             err = hipErrorInvalidValue;
             return true;
         }
-        err = mma_shape<FMT, T, true, Epi>(s, c, e, M, p);
+        err = c.xp ? mma_shape<FMT, T, true, true, Epi>(s, c, e, M, p)
+                   : mma_shape<FMT, T, true, false, Epi>(s, c, e, M, p);
         return true;
     });
 }
@@ -1175,10 +1198,12 @@ template <typename T> bool mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfm
 // gemv_mmx_kernel and gemv_rows_kernel: the 16 bytes lane l = 16 q + (m % 16)
 // supplies to k-slice s of quad qa for row tile m / 16 at u32x4 ((m / 16 quads
 // + qa) SPQ + s) 64 + l.  The grid covers the rows up to the next multiple of
-// 16; rows past M are zeros.
+// 16; rows past M are zeros.  by_row: as the staging kernel's LDS rows instead,
+// octet after octet.
 template <int FMT, typename T>
 __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_stride, const T* nw, float eps,
-                                                        uint32_t K, uint32_t M, uint32_t* out, float* part) {
+                                                        uint32_t K, uint32_t M, uint32_t* out, float* part,
+                                                        uint32_t by_row) {
     // one octet per thread (blockDim.x >= K / 8), x and w read once
     __shared__ float red[1024 / WAVE];
     const uint32_t m = blockIdx.x, KO = K / 8, cc = threadIdx.x;
@@ -1202,6 +1227,10 @@ __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_s
     if (raw && threadIdx.x < 4) part[4 * m + threadIdx.x] = threadIdx.x == 0 ? t : 0.0f;
     if (!live) return;
     const u32x4 pk = octet_scaled<FMT, T>(xv, nv, raw ? 1.0f : rr);
+    if (by_row) {
+        if (m < M) reinterpret_cast<u32x4*>(out + (size_t)m * (K / 2))[cc] = pk;
+        return;
+    }
     // octet cc of quad qa: chunk ch, pair offset 4 p4 of the chunk; k-slice sl
     // and lane group lg with mma_slice_pos(sl, lg) = (ch, 4 p4)
     using P = Mma<FMT, T>;
@@ -1219,7 +1248,7 @@ __global__ __launch_bounds__(1024) void mma_pack_kernel(const T* x, uint32_t x_s
 }  // namespace
 
 hipError_t launch_mma_pack(hipStream_t s, const void* x, uint32_t x_stride, const void* norm_w, float eps,
-                           uint32_t M, uint32_t K, int wfmt, int act, void* out, float* part) {
+                           uint32_t M, uint32_t K, int wfmt, int act, void* out, float* part, bool by_row) {
     if (M == 0 || K > 8192 || (uintptr_t)x % 16 || (x_stride * 2u) % 16 || (uintptr_t)norm_w % 16 || (uintptr_t)out % 16)
         return hipErrorInvalidValue;
     if (part && (wfmt != LSSM_W_Q4_G64 || act != LSSM_BF16)) return hipErrorInvalidValue;
@@ -1232,7 +1261,7 @@ hipError_t launch_mma_pack(hipStream_t s, const void* x, uint32_t x_stride, cons
             if (K % Mma<FMT, T>::QK != 0) return false;
             mma_pack_kernel<FMT, T><<<(M + 15) / 16 * 16, nt, 0, s>>>(
                 static_cast<const T*>(x), x_stride, static_cast<const T*>(norm_w), eps, K, M,
-                static_cast<uint32_t*>(out), part);
+                static_cast<uint32_t*>(out), part, by_row);
             err = hipGetLastError();
             return true;
         });
@@ -1271,6 +1300,12 @@ uint64_t gemv_mma_staged(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) 
     if (act == LSSM_F16) plan(f16{});
     else if (act == LSSM_BF16) plan(bf16{});
     return v;
+}
+
+bool gemv_mma_packed_pays(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) {
+    if (M < 8 || M > 14 || K > 8192 || gemv_mmx_takes(M, N, K, wfmt, act)) return false;
+    const uint64_t staged = gemv_mma_staged(M, N, K, wfmt, act);
+    return staged > 25600 && staged == (uint64_t)M * K;        // (one round of blocks)
 }
 
 bool gemv_mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act) {

@@ -436,7 +436,7 @@ bool gemv_mma_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
 // sums by 1 / rms (GemvArgs::xpart); rows up to ceil(M / 16) * 16.
 hipError_t launch_mma_pack(hipStream_t s, const void* x, uint32_t x_stride, const void* norm_w,
                            float eps, uint32_t M, uint32_t K, int wfmt, int act, void* out,
-                           float* part = nullptr);
+                           float* part = nullptr, bool by_row = false);
 // The MFMA decode GEMV takes (M, N, K) in its single-pass form, which reads x
 // packed in fragment order (launch_mma_pack).
 bool gemv_mmx_takes(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
@@ -456,6 +456,11 @@ bool gemv_rows_pays(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
 // x values the staging MFMA kernel (launch_gemv_mma without xpack) stages per
 // CU for this call when one pass takes all rows; 0 where it does not.
 uint64_t gemv_mma_staged(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
+// Whether the staging MFMA kernel is the fastest way to take a decode linear of
+// M rows packed by launch_mma_pack by_row (GemvArgs::xpack, not xrows): 8 to 14 rows in
+// one round of blocks, which hold all their weights in flight; fewer are
+// normalised in its blocks, more are read straight from memory by gemv_rows.
+bool gemv_mma_packed_pays(uint32_t M, uint32_t N, uint32_t K, int wfmt, int act);
 // Whether the VALU GEMV of up to four rows (gemv1) has this K and format.
 bool gemv1_takes(uint32_t K, int wfmt, int act);
 bool launch_gemv_rows(hipStream_t s, const GemvArgs& a, hipError_t& err);

@@ -269,6 +269,30 @@ def test_engine_unaligned_weights_decode(ctx, act, wfmt, B):
         eng.close()
 
 
+@pytest.mark.parametrize("act,wfmt", [(O.F16, O.W_Q8_G32), (O.F16, O.W_Q4_G64), (O.BF16, O.W_Q4_B32), (O.F16, O.W_DENSE)])
+@pytest.mark.parametrize("B", [7, 8, 14, 15])
+def test_engine_2p7b_widths_packed_for_staging(ctx, act, wfmt, B):
+    """2.7B layer widths at both ends of the 8 to 14 rows whose linears copy
+    packed x into the staging MFMA GEMV, and one row outside them on each side."""
+    from lite_ssm_amd.model import Engine
+    print(f"case: 2.7B widths act {act} fmt {wfmt} batch {B}", flush=True)
+    L, sh, m, om = _setup(ctx, "mamba2-2.7b", act, wfmt, n_layer=1, vocab_size=512, seed=31)
+    eng = Engine(ctx, m, max_batch=B, max_seq=4)
+    try:
+        ids = np.random.default_rng(8).integers(0, sh.vocab_size, (B, 4)).astype(np.int32)
+        nxt = torch.zeros(B, dtype=torch.int32, device="cuda")
+        eng.prefill(torch.from_numpy(ids).cuda(), nxt)
+        conv, ssd = om.new_state(B)
+        tok = O.argmax(om.prefill(conv, ssd, ids), act)
+        for step in range(2):
+            eng.decode(torch.from_numpy(tok).cuda(), nxt)
+            ref = om.decode(conv, ssd, tok)
+            _check_logits(eng.logits(B).float().cpu().numpy(), ref, act, f"2.7B widths b{B} decode {step}")
+            tok = O.argmax(ref, act)
+    finally:
+        eng.close()
+
+
 @pytest.mark.parametrize("B", [8, 24])
 def test_engine_8b_widths_packed_decode(ctx, B):
     """8B layer widths (d_model 4096, in_proj 18560 rows, G 8) at decode batches
